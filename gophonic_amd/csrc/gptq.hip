@@ -5,11 +5,10 @@
 //
 //   factor: H = X^T X over the calibration rows; dead channels (H[i][i] == 0)
 //     get H[i][i] = 1; H += 0.01 * mean(diag) * I; U = J chol(J H J)^-1 J, the
-//     upper factor with H^-1 = U^T U. The Cholesky factorization runs in
-//     64-column panels (diagonal block in one workgroup with float64 sums,
-//     panel rows by forward substitution, the trailing update as an fp32
-//     product); L^-1 runs in 64-row blocks (an fp32 product with the rows
-//     already inverted, then the block's rows by substitution).
+//     upper factor with H^-1 = U^T U. The factorization and the factor's
+//     inverse advance together in 64-column panels, two launches each (the
+//     diagonal block and the products with its inverse in float64, the
+//     trailing products fp32).
 //   round: per 128-column block, one wavefront per weight row quantizes the
 //     block's columns in order (code = clamp(rne(w / s)), error
 //     e = (w - q s) / U[c][c], the block's later columns w[j] -= e U[c][j]),
@@ -35,204 +34,450 @@ constexpr int kRowsPerBlock = 8;  // weight rows (wavefronts) per rounding workg
 
 // ---- fp32 product: C = [C +] alpha * op(A) op(B) ---------------------------
 // A(i,p) = a[i*lda + p] (TA 0) or a[p*lda + i] (TA 1); B(p,j) = b[p*ldb + j]
-// (TB 0) or b[j*ldb + p] (TB 1). 64 x 64 tiles, 256 threads with 4 x 4
-// outputs each, 16-deep K chunks through LDS. lower: only j <= i is written.
-// With accumulate the full sum is formed first and added once.
-template <int TA, int TB>
-__global__ __launch_bounds__(256) void sgemm_kernel(int M, int N, int K, float alpha, const float *__restrict__ a,
-                                                    long lda, const float *__restrict__ b, long ldb, float *c,
-                                                    long ldc, int accumulate, int lower) {
-    __shared__ float As[16][68], Bs[16][68];
-    const int bi = blockIdx.y * 64, bj = blockIdx.x * 64;
-    if (lower && bj > bi + 63) return;
-    const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
-    float acc[4][4] = {};
-    for (int p0 = 0; p0 < K; p0 += 16) {
+// (TB 0) or b[j*ldb + p] (TB 1). BM x BN tiles, four wavefronts as 2 x 2, each
+// on 32 x 32 tiles of v_mfma_f32_32x32x2_f32 (fp32 products and sums). 16-deep
+// K chunks, double-buffered in LDS, the next chunk's loads in flight during
+// the MFMAs, one barrier per chunk. An operand whose memory runs along K lies
+// in LDS as [i][16 + 4] (one 16-byte read feeds four MFMAs), the other kind as
+// [p][BM + 8] (four 4-byte reads); both conflict-free. Of each 8 K values lane
+// half h multiplies 4h .. 4h + 3, so an MFMA pairs p with p + 4. With
+// accumulate the full sum is formed first and added once.
+using f32x16 = __attribute__((ext_vector_type(16))) float;
+
+enum SgemmMode {
+    kFull,
+    // j >= i only, stored at C[M-1-i][N-1-j]: the Gram matrix J H J, its lower
+    // triangle (M == N).
+    kUpperReversed,
+};
+
+struct SgemmArgs {
+    int M, N, K;
+    float alpha;
+    const float *a, *b;
+    float *c;
+    long lda, ldb, ldc;
+    int accumulate;
+    int vecA, vecB;  // 16-byte loads: base aligned, stride a multiple of 4
+};
+
+inline int vec16(const float *p, long ld) { return ((uintptr_t)p % 16 == 0 && ld % 4 == 0) ? 1 : 0; }
+
+// Rows [i0, i0 + BM) x K chunk [p0, p0 + 16) of an operand with `rows` rows and
+// K values, as BM/64 float4 per thread; zero past the edges.
+template <int T, int BM>
+__device__ __forceinline__ void sgemm_fetch(float4 (&v)[BM / 64], const float *x, long ld, int rows, int K, int i0,
+                                            int p0, bool vec) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int idx = t + 256 * e;
-            int i, p, j, q;
-            if (TA == 0) {
-                i = idx >> 4;
-                p = idx & 15;
+    for (int e = 0; e < BM / 64; ++e) {
+        const int idx = (int)threadIdx.x + 256 * e;
+        const int i = i0 + (T == 0 ? idx >> 2 : (idx % (BM / 4)) * 4);
+        const int p = p0 + (T == 0 ? (idx & 3) * 4 : idx / (BM / 4));
+        const int left = T == 0 ? (i < rows ? K - p : 0) : (p < K ? rows - i : 0);
+        float r[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (left > 0) {
+            const float *src = T == 0 ? x + (size_t)i * ld + p : x + (size_t)p * ld + i;
+            if (vec && left >= 4) {
+                const float4 q = *(const float4 *)src;
+                r[0] = q.x, r[1] = q.y, r[2] = q.z, r[3] = q.w;
             } else {
-                p = idx >> 6;
-                i = idx & 63;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    if (d < left) r[d] = src[d];
             }
-            float va = 0.0f;
-            if (bi + i < M && p0 + p < K)
-                va = TA == 0 ? a[(size_t)(bi + i) * lda + p0 + p] : a[(size_t)(p0 + p) * lda + bi + i];
-            As[p][i] = va;
-            if (TB == 0) {
-                q = idx >> 6;
-                j = idx & 63;
-            } else {
-                j = idx >> 4;
-                q = idx & 15;
-            }
-            float vb = 0.0f;
-            if (bj + j < N && p0 + q < K)
-                vb = TB == 0 ? b[(size_t)(p0 + q) * ldb + bj + j] : b[(size_t)(bj + j) * ldb + p0 + q];
-            Bs[q][j] = vb;
         }
-        __syncthreads();
-#pragma unroll
-        for (int p = 0; p < 16; ++p) {
-            float x[4], y[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                x[r] = As[p][ty * 4 + r];
-                y[r] = Bs[p][tx * 4 + r];
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int s = 0; s < 4; ++s) acc[r][s] = fmaf(x[r], y[s], acc[r][s]);
-        }
-        __syncthreads();
+        v[e] = make_float4(r[0], r[1], r[2], r[3]);
     }
+}
+
+template <int T, int BM>
+__device__ __forceinline__ void sgemm_stash(float *lds, const float4 (&v)[BM / 64]) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int e = 0; e < BM / 64; ++e) {
+        const int idx = (int)threadIdx.x + 256 * e;
+        float *d = T == 0 ? lds + (idx >> 2) * 20 + (idx & 3) * 4
+                          : lds + (idx / (BM / 4)) * (BM + 8) + (idx % (BM / 4)) * 4;
+        *(float4 *)d = v[e];
+    }
+}
+
+// Four MFMAs' operand values of one 32-row tile: K values 8g + 4h .. + 3 of row i.
+template <int T, int BM>
+__device__ __forceinline__ void sgemm_frag(float (&f)[4], const float *lds, int i, int g, int h) {
+    if (T == 0) {
+        const float4 q = *(const float4 *)(lds + i * 20 + g * 8 + h * 4);
+        f[0] = q.x, f[1] = q.y, f[2] = q.z, f[3] = q.w;
+    } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int i = bi + ty * 4 + r, j = bj + tx * 4 + s;
-            if (i >= M || j >= N || (lower && j > i)) continue;
-            const float v = alpha * acc[r][s];
-            float *p = c + (size_t)i * ldc + j;
-            *p = accumulate ? *p + v : v;
+        for (int e = 0; e < 4; ++e) f[e] = lds[(g * 8 + h * 4 + e) * (BM + 8) + i];
+    }
+}
+
+// LDS floats of one K chunk of an operand of kind T (0: runs along K).
+template <int T, int BM>
+constexpr int sgemm_lds() {
+    return T == 0 ? BM * 20 : 16 * (BM + 8);
+}
+
+// The lower-triangle pair (row >= col) numbered t, row by row.
+__device__ __forceinline__ void tri_pair(int t, int &row, int &col) {
+    row = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+    while ((long)row * (row + 1) / 2 > t) --row;
+    while ((long)(row + 1) * (row + 2) / 2 <= t) ++row;
+    col = t - (int)((long)row * (row + 1) / 2);
+}
+
+template <int TA, int TB, int BM, int BN, int MODE>
+__global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
+    constexpr int MT = BM / 64, NT = BN / 64;  // 32 x 32 tiles per wavefront
+    __shared__ __attribute__((aligned(16))) float As[2][sgemm_lds<TA, BM>()], Bs[2][sgemm_lds<TB ^ 1, BN>()];
+    const int M = g.M, N = g.N, K = g.K;
+    int ti, tj;
+    if (MODE == kUpperReversed) {
+        tri_pair((int)blockIdx.x, tj, ti);
+    } else {
+        const int tn = (N + BN - 1) / BN;
+        ti = (int)blockIdx.x / tn;
+        tj = (int)blockIdx.x - ti * tn;
+    }
+    const int bi = ti * BM, bj = tj * BN;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, h = lane >> 5;
+    const int wi = (wave >> 1) * (BM / 2), wj = (wave & 1) * (BN / 2);
+    f32x16 acc[MT][NT] = {};
+    float4 va[BM / 64], vb[BN / 64];
+    sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, 0, g.vecA);
+    sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, 0, g.vecB);
+    sgemm_stash<TA, BM>(As[0], va);
+    sgemm_stash<TB ^ 1, BN>(Bs[0], vb);
+    __syncthreads();
+    int buf = 0;
+    for (int p0 = 0; p0 < K; p0 += 16) {
+        const bool more = p0 + 16 < K;
+        if (more) {
+            sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, p0 + 16, g.vecA);
+            sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, p0 + 16, g.vecB);
         }
+#pragma unroll
+        for (int gr = 0; gr < 2; ++gr) {
+            float fa[MT][4], fb[NT][4];
+#pragma unroll
+            for (int x = 0; x < MT; ++x) sgemm_frag<TA, BM>(fa[x], As[buf], wi + 32 * x + li, gr, h);
+#pragma unroll
+            for (int y = 0; y < NT; ++y) sgemm_frag<TB ^ 1, BN>(fb[y], Bs[buf], wj + 32 * y + li, gr, h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int x = 0; x < MT; ++x)
+#pragma unroll
+                    for (int y = 0; y < NT; ++y)
+                        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[x][e], fb[y][e], acc[x][y], 0, 0, 0);
+        }
+        if (more) {
+            sgemm_stash<TA, BM>(As[buf ^ 1], va);
+            sgemm_stash<TB ^ 1, BN>(Bs[buf ^ 1], vb);
+        }
+        __syncthreads();
+        buf ^= 1;
+    }
+    // Result register r of lane l: row (r & 3) + 8 (r >> 2) + 4 h, column l % 32.
+#pragma unroll
+    for (int x = 0; x < MT; ++x)
+#pragma unroll
+        for (int y = 0; y < NT; ++y)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int i = bi + wi + 32 * x + (r & 3) + 8 * (r >> 2) + 4 * h, j = bj + wj + 32 * y + li;
+                if (i >= M || j >= N) continue;
+                const float v = g.alpha * acc[x][y][r];
+                if (MODE == kUpperReversed) {
+                    if (j >= i) g.c[(size_t)(M - 1 - i) * g.ldc + (N - 1 - j)] = v;
+                } else {
+                    float *p = g.c + (size_t)i * g.ldc + j;
+                    *p = g.accumulate ? *p + v : v;
+                }
+            }
 }
 
 template <int TA, int TB>
 int sgemm(int M, int N, int K, float alpha, const float *a, long lda, const float *b, long ldb, float *c, long ldc,
-          bool accumulate, bool lower, hipStream_t st) {
+          bool accumulate, hipStream_t st) {
     if (M <= 0 || N <= 0) return GPHQ_OK;
-    hipLaunchKernelGGL((sgemm_kernel<TA, TB>), dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64)),
-                       dim3(256), 0, st, M, N, K, alpha, a, lda, b, ldb, c, ldc, accumulate ? 1 : 0, lower ? 1 : 0);
+    const SgemmArgs g{M, N, K, alpha, a, b, c, lda, ldb, ldc, accumulate ? 1 : 0, vec16(a, lda), vec16(b, ldb)};
+    // 128 x 128 tiles halve the operand reads; below two rounds of the chip
+    // the 64 x 64 tiles' four times as many blocks matter more.
+    const long big = (long)((M + 127) / 128) * ((N + 127) / 128);
+    if (big >= 2L * device_cus())
+        hipLaunchKernelGGL((sgemm_kernel<TA, TB, 128, 128, kFull>), dim3((unsigned)big), dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((sgemm_kernel<TA, TB, 64, 64, kFull>),
+                           dim3((unsigned)((M + 63) / 64) * (unsigned)((N + 63) / 64)), dim3(256), 0, st, g);
     return launch_status();
 }
 
-// Dead channels and damping (gptq.go:623-637): one block; the diagonal's mean
-// in float64.
-__global__ __launch_bounds__(1024) void gptq_damp_kernel(float *h, int n, uint8_t *dead) {
+// Dead channels and damping (gptq.go:623-637) on A = J H J (A[i][i] is channel
+// n-1-i): one block; the diagonal's mean in float64. Clears *bad.
+__global__ __launch_bounds__(1024) void gptq_damp_kernel(float *a, int n, uint8_t *dead, int *bad) {
     __shared__ double part[16];
     double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += (double)h[(size_t)i * n + i];
+    for (int i = threadIdx.x; i < n; i += blockDim.x) s += (double)a[(size_t)i * n + i];
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+    if (threadIdx.x == 0) *bad = 0;
     __syncthreads();
     double mean = 0.0;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mean += part[w];
     mean /= (double)n;
     const float add = (float)(0.01 * mean);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        float d = h[(size_t)i * n + i];
+        float d = a[(size_t)i * n + i];
         const bool isDead = d == 0.0f;
-        dead[i] = isDead ? 1 : 0;
+        dead[n - 1 - i] = isDead ? 1 : 0;
         if (isDead) d = 1.0f;
-        h[(size_t)i * n + i] = d + add;
+        a[(size_t)i * n + i] = d + add;
     }
 }
 
-// dst = J src J (both n x n): dst[i][j] = src[n-1-i][n-1-j].
-__global__ void reverse_kernel(const float *__restrict__ src, float *__restrict__ dst, int n) {
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (size_t)n * n) return;
-    const int i = (int)(idx / n), j = (int)(idx - (size_t)i * n);
-    dst[idx] = src[(size_t)(n - 1 - i) * n + (n - 1 - j)];
-}
+// ---- Cholesky of A = J H J and the inverse of its factor ---------------------
+// What the factor of an n x n matrix cannot do without is n^3 multiply-adds
+// (half of H, a third each for L and L^-1), but its columns form a chain, one
+// step per 64-column panel. Both factors advance in the same step, as an
+// elimination on [A | I], so a step is two launches whatever n: with the
+// diagonal block's inverse at hand chol_panel_kernel forms the panel below the
+// block and the inverse's rows beside it (products in float64, where a
+// substitution would be 64 dependent divisions), and chol_update_kernel takes
+// the panel's products off the trailing tiles of A and adds them to the sums
+// S = L X of the inverse's later rows. Its first block, which owns the next
+// diagonal block, goes on to factor and invert that block while the others
+// update. X's rows come from the sums over all rows above them, as in a
+// substitution, so L X = I holds to fp32 rounding of |L||X| (products of
+// inverted blocks, X21 = -X22 (L21 X11), have no such bound). K = 4096 from
+// 4096 rows: 53.5 -> 5.56 ms (separate launches for the block, the panel's
+// substitution and the update, then one thin product and a substitution per 64
+// rows of the inverse, took 84 + 207 + 21 + 357 + 137 us a panel).
 
-// Factors the b x b diagonal block at j0 (already updated by earlier panels)
-// in place, choleskyLower's inner loop (gptq_linalg.go:73-93): float64 sums,
-// float64 pivot roots, float32 storage. Sets *bad on a non-positive pivot.
-__global__ __launch_bounds__(64) void chol_diag_kernel(float *a, int n, int j0, int b, int *bad) {
-    __shared__ float L[kPanel][kPanel + 1];
-    __shared__ double piv;
-    const int t = threadIdx.x;
-    if (t < b)
-        for (int p = 0; p <= t; ++p) L[t][p] = a[(size_t)(j0 + t) * n + j0 + p];
-    __syncthreads();
-    for (int j = 0; j < b; ++j) {
-        if (t == j) {
-            double d = 0.0;
-            for (int p = 0; p < j; ++p) d += (double)L[j][p] * (double)L[j][p];
-            d = (double)L[j][j] - d;
-            if (!(d > 0.0)) {
-                *bad = 1;
-                d = 1.0;
+// The packed lower triangle of a 64 x 64 block: row r, column c <= r.
+__device__ __forceinline__ int packed(int r, int c) { return r * (r + 1) / 2 + c; }
+
+// Factors the b x b (b <= 64) diagonal block held in S (lower triangle) and
+// inverts the factor, with 256 threads: choleskyLower's inner loop
+// (gptq_linalg.go:73-93) with float64 sums and pivot roots, L rounded to
+// float32 as it is formed. L goes to l (row stride ld), L^-1 to x as float32
+// (row stride ld) and, unless inv is null (no panel follows), to inv as packed
+// float64 for the panel product. Thread
+// (i, q) holds columns 4k + q of row i of the block and of the inverse, which
+// starts as the identity and takes the same row operations. Each of the 64
+// steps costs a float64 root and reciprocal, one LDS exchange and one barrier:
+// a chain of 52 us, longer than the other blocks' update beside it.
+__device__ void chol_diag(const float (*S)[65], double (*col)[64], float (*Ls)[65], int b, float *l, float *x,
+                          long ld, double *inv, int *bad) {
+    const int i = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    double a[16], w[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const int c = 4 * k + q;
+        // Past b the block continues as the identity.
+        a[k] = i < b ? (c <= i ? (double)S[i][c] : 0.0) : (c == i ? 1.0 : 0.0);
+        w[k] = c == i ? 1.0 : 0.0;
+    }
+    const auto lane_of = [](double v, int from) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, from);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), from);
+        return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+    };
+#pragma unroll
+    for (int k0 = 0; k0 < 16; ++k0)
+#pragma unroll 1
+        for (int jj = 0; jj < 4; ++jj) {
+            const int j = 4 * k0 + jj;
+            if (q == jj) {  // this wavefront holds column j
+                double d = lane_of(a[k0], j);
+                if (!(d > 0.0)) {
+                    if (i == 0 && j < b) *bad = 1;
+                    d = 1.0;
+                }
+                const double piv = sqrt(d);
+                const float v = i == j ? (float)piv : i > j ? (float)(a[k0] / piv) : 0.0f;
+                Ls[i][j] = v;
+                col[j & 1][i] = (double)v;
             }
-            piv = sqrt(d);
-            L[j][j] = (float)piv;
+            __syncthreads();
+            const double *cj = col[j & 1];
+            const double li = cj[i], ljj = 1.0 / cj[j];
+            // Rows past j lose L[i][j] times row j; row j of the inverse is scaled.
+            const double f = i > j ? li : 0.0;
+#pragma unroll
+            for (int k = k0; k < 16; ++k) a[k] -= f * cj[4 * k + q];
+#pragma unroll
+            for (int k = 0; k <= k0; ++k) {
+                const double xj = lane_of(w[k], j) * ljj;
+                w[k] = i == j ? xj : w[k] - f * xj;
+            }
         }
-        __syncthreads();
-        if (t > j && t < b) {
-            double s = 0.0;
-            for (int p = 0; p < j; ++p) s += (double)L[t][p] * (double)L[j][p];
-            L[t][j] = (float)(((double)L[t][j] - s) / piv);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const int c = 4 * k + q;
+        if (i < b && c <= i) {
+            x[(size_t)i * ld + c] = (float)w[k];
+            if (inv) inv[packed(i, c)] = w[k];
         }
-        __syncthreads();
     }
-    if (t < b)
-        for (int p = 0; p <= t; ++p) a[(size_t)(j0 + t) * n + j0 + p] = L[t][p];
+    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
+        const int r = e >> 6, c = e & 63;
+        if (r < b && c <= r) l[(size_t)r * ld + c] = Ls[r][c];
+    }
 }
 
-// Panel rows below the diagonal block: L21 = A21 L11^-T row by row
-// (gptq_linalg.go:97-110), one thread per row, float64 sums.
-__global__ __launch_bounds__(256) void chol_panel_kernel(float *a, int n, int j0, int b) {
-    __shared__ float L[kPanel][kPanel + 1];
-    for (int e = threadIdx.x; e < b * b; e += blockDim.x) {
-        const int r = e / b, p = e - r * b;
-        L[r][p] = p <= r ? a[(size_t)(j0 + r) * n + j0 + p] : 0.0f;
+struct DiagLds {
+    float S[64][65], Ls[64][65];
+    double col[2][64];
+};
+
+// The first diagonal block.
+__global__ __launch_bounds__(256) void chol_first_kernel(float *a, int n, float *x, double *inv, int *bad) {
+    __shared__ DiagLds d;
+    const int b = min(64, n);
+    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
+        const int r = e >> 6, c = e & 63;
+        d.S[r][c] = r < b && c <= r ? a[(size_t)r * n + c] : 0.0f;
     }
     __syncthreads();
-    const int i = j0 + b + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= n) return;
-    float *row = a + (size_t)i * n + j0;
-    float v[kPanel];
-#pragma unroll
-    for (int j = 0; j < kPanel; ++j) v[j] = j < b ? row[j] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < kPanel; ++j) {
-        if (j >= b) break;
-        double s = (double)v[j];
-#pragma unroll
-        for (int p = 0; p < kPanel; ++p)
-            if (p < j) s -= (double)v[p] * (double)L[j][p];
-        v[j] = (float)(s / (double)L[j][j]);
-    }
-#pragma unroll
-    for (int j = 0; j < kPanel; ++j)
-        if (j < b) row[j] = v[j];
+    chol_diag(d.S, d.col, d.Ls, b, a, x, n, inv, bad);
 }
 
-// Rows i0 .. i0+b-1 of X = L^-1 (lower), every column c <= i: X[i][c] =
-// (delta(i,c) - sum_{p<i} L[i][p] X[p][c]) / L[i][i], the part p < i0 given
-// as T[r][c] (an fp32 product), the rest summed here in float64 over the
-// block's earlier rows (invertLowerTransposed, gptq_linalg.go:141-176). One
-// thread per column; X's columns of the block's rows kept in LDS.
-__global__ __launch_bounds__(256) void inv_rows_kernel(const float *__restrict__ l, float *__restrict__ x,
-                                                       const float *__restrict__ tt, int n, int i0, int b) {
-    __shared__ float Lb[kPanel][kPanel + 1];
-    __shared__ float xs[kPanel][256];
-    for (int e = threadIdx.x; e < b * b; e += blockDim.x) {
-        const int r = e / b, p = e - r * b;
-        Lb[r][p] = p <= r ? l[(size_t)(i0 + r) * n + i0 + p] : 0.0f;
+using f64x4 = __attribute__((ext_vector_type(4))) double;
+
+// The step at j0, on v_mfma_f64_16x16x4_f64. Blocks below `below`: 32 panel
+// rows each, L21 = A21 L11^-T (gptq_linalg.go:97-110). The others: 32 columns
+// each of the inverse's rows j0 .. j0+63, X = -L11^-1 S.
+__global__ __launch_bounds__(256) void chol_panel_kernel(float *a, float *x, int n, int j0, int below,
+                                                         const double *__restrict__ inv) {
+    __shared__ double Li[64][66];  // L11^-1, zero above the diagonal
+    __shared__ float Ar[64][36];   // the panel's 32 rows as [p][row], or S's 32 columns as [p][column]
+    const bool rows = (int)blockIdx.x < below;
+    const int i0 = rows ? j0 + 64 + (int)blockIdx.x * 32 : ((int)blockIdx.x - below) * 32;
+    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
+        const int r = e >> 6, c = e & 63;
+        Li[r][c] = c <= r ? inv[packed(r, c)] : 0.0;
+    }
+    for (int e = threadIdx.x; e < 32 * 64; e += 256) {
+        if (rows) {
+            const int r = e >> 6, c = e & 63;
+            Ar[c][r] = i0 + r < n ? a[(size_t)(i0 + r) * n + j0 + c] : 0.0f;
+        } else {
+            const int r = e >> 5, c = e & 31;
+            Ar[r][c] = j0 + r < n ? x[(size_t)(j0 + r) * n + i0 + c] : 0.0f;
+        }
     }
     __syncthreads();
-    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (c >= i0 + b) return;
-    for (int r = 0; r < b; ++r) {
-        const int i = i0 + r;
-        float v = 0.0f;
-        if (c <= i) {
-            double s = c < i0 ? (double)tt[(size_t)r * i0 + c] : 0.0;
-            for (int p = max(0, c - i0); p < r; ++p) s += (double)Lb[r][p] * (double)xs[p][threadIdx.x];
-            const double num = c == i ? 1.0 : -s;
-            v = (float)(num / (double)Lb[r][r]);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    // Wavefront w: L11^-1's rows 16w .. 16w+15, which need p <= 16w + 15.
+    f64x4 acc[2] = {};
+    for (int p = 0; p < 16 * (wave + 1); p += 4) {
+        const double lv = Li[16 * wave + li][p + lk];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const double v = (double)Ar[p + lk][16 * t + li];
+            acc[t] = rows ? __builtin_amdgcn_mfma_f64_16x16x4f64(v, lv, acc[t], 0, 0, 0)
+                          : __builtin_amdgcn_mfma_f64_16x16x4f64(lv, v, acc[t], 0, 0, 0);
         }
-        xs[r][threadIdx.x] = v;
-        x[(size_t)i * n + c] = v;
     }
+    // Result register r of lane l: row 4 r + l / 16, column l % 16.
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (rows) {
+                const int i = i0 + 16 * t + 4 * r + lk;
+                if (i < n) a[(size_t)i * n + j0 + 16 * wave + li] = (float)acc[t][r];
+            } else {
+                const int i = j0 + 16 * wave + 4 * r + lk;
+                if (i < n) x[(size_t)i * n + i0 + 16 * t + li] = (float)-acc[t][r];
+            }
+        }
+}
+
+// The rest of the step at j0, in 64 x 64 tiles (fp32 products and sums, the
+// whole 64-deep sum added once). Blocks below `tri`: A22 -= L21 L21^T on the
+// lower triangle; block 0 then factors and inverts the diagonal block it has
+// just updated, the next step's. The others: S += L21 X[j0 .. j0+63], the
+// columns of the diagonal block for the first time.
+__global__ __launch_bounds__(256) void chol_update_kernel(float *a, int n, int j0, int tri, float *x, double *inv,
+                                                          int *bad, int vec) {
+    __shared__ union {
+        struct {
+            __attribute__((aligned(16))) float A[64][68], B[64][72];
+        } p;
+        DiagLds d;
+    } sh;
+    const int j1 = j0 + 64;
+    const bool trailing = (int)blockIdx.x < tri;
+    int ti, tj;
+    if (trailing) {
+        tri_pair((int)blockIdx.x, ti, tj);
+    } else {
+        const int cols = j1 / 64, t = (int)blockIdx.x - tri;
+        ti = t / cols;
+        tj = t - ti * cols;
+    }
+    const int bi = j1 + ti * 64, bj = trailing ? j1 + tj * 64 : tj * 64;
+    float *const c = trailing ? a : x;
+    const bool fresh = !trailing && bj == j0;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, h = lane >> 5;
+    const int wi = (wave >> 1) * 32, wj = (wave & 1) * 32;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int idx = (int)threadIdx.x + 256 * e, r = idx >> 4, q = (idx & 15) * 4;
+        float4 va = make_float4(0, 0, 0, 0), vb = va;
+        const float *pa = a + (size_t)(bi + r) * n + j0 + q;
+        if (bi + r < n) va = vec ? *(const float4 *)pa : make_float4(pa[0], pa[1], pa[2], pa[3]);
+        // L21's rows [j][p], or the inverse's rows [p][j] (its diagonal block is lower).
+        const float *pb = trailing ? a + (size_t)(bj + r) * n + j0 + q : x + (size_t)(j0 + r) * n + bj + q;
+        if (!trailing || bj + r < n) vb = vec ? *(const float4 *)pb : make_float4(pb[0], pb[1], pb[2], pb[3]);
+        if (fresh)
+            vb = make_float4(q <= r ? vb.x : 0.0f, q + 1 <= r ? vb.y : 0.0f, q + 2 <= r ? vb.z : 0.0f,
+                             q + 3 <= r ? vb.w : 0.0f);
+        *(float4 *)&sh.p.A[r][q] = va;
+        *(float4 *)&sh.p.B[r][q] = vb;
+    }
+    // The tile's own values, in flight during the product.
+    float own[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int i = bi + wi + (r & 3) + 8 * (r >> 2) + 4 * h, j = bj + wj + li;
+        own[r] = i < n && j <= i && !fresh ? c[(size_t)i * n + j] : 0.0f;
+    }
+    __syncthreads();
+    f32x16 acc = {};
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+        const float4 fa = *(const float4 *)&sh.p.A[wi + li][8 * g + 4 * h];
+        float4 fb;
+        if (trailing) {
+            fb = *(const float4 *)&sh.p.B[wj + li][8 * g + 4 * h];
+        } else {
+            const float *b = &sh.p.B[8 * g + 4 * h][wj + li];
+            fb = make_float4(b[0], b[72], b[144], b[216]);
+        }
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa.x, fb.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa.y, fb.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa.z, fb.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa.w, fb.w, acc, 0, 0, 0);
+    }
+    const bool diag = blockIdx.x == 0;
+    if (diag) __syncthreads();  // every wavefront has read its operands
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int lr = wi + (r & 3) + 8 * (r >> 2) + 4 * h, lc = wj + li;
+        const float v = trailing ? own[r] - acc[r] : own[r] + acc[r];
+        if (diag) sh.d.S[lr][lc] = v;
+        else if (bi + lr < n && bj + lc <= bi + lr) c[(size_t)(bi + lr) * n + bj + lc] = v;
+    }
+    if (!diag) return;
+    __syncthreads();
+    chol_diag(sh.d.S, sh.d.col, sh.d.Ls, min(64, n - j1), a + (size_t)j1 * n + j1, x + (size_t)j1 * n + j1, n, inv,
+              bad);
 }
 
 // U[r][c] = X[n-1-r][n-1-c] for c >= r, else 0 (gptq_linalg.go:208-221).
@@ -415,7 +660,7 @@ namespace gphq {
 // product). The calibration pass's projections and residual adds.
 int sgemm_abt(int M, int N, int K, const float *a, long lda, const float *b, long ldb, float *c, long ldc,
               bool accumulate, hipStream_t st) {
-    return sgemm<0, 1>(M, N, K, 1.0f, a, lda, b, ldb, c, ldc, accumulate, false, st);
+    return sgemm<0, 1>(M, N, K, 1.0f, a, lda, b, ldb, c, ldc, accumulate, st);
 }
 
 }  // namespace gphq
@@ -434,43 +679,41 @@ int gphq_gptq_factor(const float *x_dev, int64_t rows, int64_t k, float *u_dev, 
     if (work_bytes < gphq_gptq_work_bytes(k)) return GPHQ_ERR_DIMENSIONS;
     hipStream_t st = (hipStream_t)stream;
     const int n = (int)k;
-    float *h = (float *)work_dev;                    // H, then X = L^-1
-    float *tt = h + (size_t)n * n;                   // [64][n]
-    int *bad = (int *)(tt + (size_t)kPanel * n);
-    GPHQ_TRY(hip_status(hipMemsetAsync(bad, 0, sizeof(int), st)));
-    // H = X^T X (gptq.go:606-622).
-    GPHQ_TRY((sgemm<1, 0>(n, n, (int)rows, 1.0f, x_dev, n, x_dev, n, h, n, false, false, st)));
-    hipLaunchKernelGGL(gptq_damp_kernel, dim3(1), dim3(1024), 0, st, h, n, dead_dev);
-    GPHQ_TRY(launch_status());
     const size_t nn = (size_t)n * n;
     const unsigned eb = (unsigned)((nn + 255) / 256);
-    // A = J H J into u_dev; lower Cholesky in place (gptq_linalg.go:68-132).
-    hipLaunchKernelGGL(reverse_kernel, dim3(eb), dim3(256), 0, st, h, u_dev, n);
-    GPHQ_TRY(launch_status());
+    float *x = (float *)work_dev;  // X = L^-1
+    // L11^-1 of the current panel: 2080 doubles (only read when n > 64, where
+    // they fit the 64 n floats here with the alignment's 4 bytes).
+    double *inv = (double *)(((uintptr_t)(x + nn) + 7) & ~(uintptr_t)7);
+    int *bad = (int *)((char *)work_dev + gphq_gptq_work_bytes(k) - 64);
     float *A = u_dev;
+    // A = J H J, H = X^T X (gptq.go:606-622), its lower triangle; dead channels and damping.
+    const SgemmArgs g{n, n, (int)rows, 1.0f, x_dev, x_dev, A, n, n, n, 0, vec16(x_dev, n), vec16(x_dev, n)};
+    const long t64 = (n + 63) / 64;
+    hipLaunchKernelGGL((sgemm_kernel<1, 0, 64, 64, kUpperReversed>), dim3((unsigned)(t64 * (t64 + 1) / 2)), dim3(256),
+                       0, st, g);
+    GPHQ_TRY(launch_status());
+    hipLaunchKernelGGL(gptq_damp_kernel, dim3(1), dim3(1024), 0, st, A, n, dead_dev, bad);
+    GPHQ_TRY(launch_status());
+    // Lower Cholesky in place (gptq_linalg.go:68-132), the inverses of the
+    // diagonal blocks into x on the way.
+    hipLaunchKernelGGL(chol_first_kernel, dim3(1), dim3(256), 0, st, A, n, x,
+                       n > kPanel ? inv : nullptr, bad);
+    GPHQ_TRY(launch_status());
     for (int j0 = 0; j0 < n; j0 += kPanel) {
-        const int b = std::min(kPanel, n - j0), j1 = j0 + b;
-        hipLaunchKernelGGL(chol_diag_kernel, dim3(1), dim3(kPanel), 0, st, A, n, j0, b, bad);
+        const int m = std::max(0, n - j0 - kPanel);
+        const int below = (m + 31) / 32, left = j0 / 32;
+        if (below + left > 0)
+            hipLaunchKernelGGL(chol_panel_kernel, dim3((unsigned)(below + left)), dim3(256), 0, st, A, x, n, j0,
+                               below, inv);
         GPHQ_TRY(launch_status());
-        if (j1 == n) break;
-        hipLaunchKernelGGL(chol_panel_kernel, dim3((unsigned)((n - j1 + 255) / 256)), dim3(256), 0, st, A, n, j0, b);
-        GPHQ_TRY(launch_status());
-        // A22 -= L21 L21^T on the lower triangle.
-        const int m = n - j1;
-        GPHQ_TRY((sgemm<0, 1>(m, m, b, -1.0f, A + (size_t)j1 * n + j0, n, A + (size_t)j1 * n + j0, n,
-                             A + (size_t)j1 * n + j1, n, true, true, st)));
-    }
-    // X = L^-1 into h (gptq_linalg.go:134-176).
-    GPHQ_TRY(hip_status(hipMemsetAsync(h, 0, nn * sizeof(float), st)));
-    for (int i0 = 0; i0 < n; i0 += kPanel) {
-        const int b = std::min(kPanel, n - i0);
-        if (i0 > 0)  // T = L[i0:i0+b][0:i0] X[0:i0][0:i0]
-            GPHQ_TRY((sgemm<0, 0>(b, i0, i0, 1.0f, A + (size_t)i0 * n, n, h, n, tt, i0, false, false, st)));
-        hipLaunchKernelGGL(inv_rows_kernel, dim3((unsigned)((i0 + b + 255) / 256)), dim3(256), 0, st, A, h, tt, n, i0,
-                           b);
+        if (m == 0) break;
+        const long tiles = (m + 63) / 64, tri = tiles * (tiles + 1) / 2;
+        hipLaunchKernelGGL(chol_update_kernel, dim3((unsigned)(tri + tiles * (j0 / 64 + 1))), dim3(256), 0, st, A, n,
+                           j0, (int)tri, x, inv, bad, vec16(A, n) & vec16(x, n));
         GPHQ_TRY(launch_status());
     }
-    hipLaunchKernelGGL(u_from_x_kernel, dim3(eb), dim3(256), 0, st, h, u_dev, n);
+    hipLaunchKernelGGL(u_from_x_kernel, dim3(eb), dim3(256), 0, st, x, u_dev, n);
     GPHQ_TRY(launch_status());
     int flag = 0;
     GPHQ_TRY(hip_status(hipMemcpyAsync(&flag, bad, sizeof(int), hipMemcpyDeviceToHost, st)));
@@ -521,7 +764,7 @@ int gphq_gptq_round(float *w_dev, int64_t n, int64_t k, const float *u_dev, cons
         GPHQ_TRY(launch_status());
         if (i2 < k)  // W[:, i2:] -= E U[i1:i2, i2:] (gptq.go:746-760)
             GPHQ_TRY((sgemm<0, 0>((int)n, (int)(k - i2), b, -1.0f, errs, kRoundBlock, u_dev + (size_t)i1 * k + i2, k,
-                                 w_dev + i2, k, true, false, st)));
+                                 w_dev + i2, k, true, st)));
     }
     return GPHQ_OK;
 }

@@ -85,6 +85,22 @@ def test_factor_meets_the_reference_bound(k):
     assert worst <= 1e-4, worst
 
 
+@pytest.mark.parametrize("k", [2, 63, 64, 65, 66, 127, 129, 191, 194, 516])
+def test_factor_at_panel_edges(k):
+    """One panel, the first step of a second, partial last panels and widths
+    whose rows are not 16-byte aligned, held to the reference's bound on its
+    well-conditioned H (as test_factor_meets_the_reference_bound)."""
+    rng = np.random.default_rng(k)
+    xs = np.vstack([rng.standard_normal((k + 3, k)) / np.sqrt(k + 3), np.eye(k)]).astype(np.float32)
+    xs[:, k // 2] = 0  # a dead channel
+    u, dead = factor(xs)
+    h, want_dead = go.damp(go.hessian(xs))
+    assert np.array_equal(dead, want_dead)
+    assert np.array_equal(u, np.triu(u))
+    u64 = u.astype(np.float64)
+    assert np.abs(h @ (u64.T @ u64) - np.eye(k)).max() <= 1e-4
+
+
 def test_factor_rejects_non_finite_hessian():
     import torch
 
