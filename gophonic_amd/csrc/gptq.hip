@@ -144,6 +144,10 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, h = lane >> 5;
     const int wi = (wave >> 1) * (BM / 2), wj = (wave & 1) * (BN / 2);
     f32x16 acc[MT][NT] = {};
+    // The Gram matrix's sums run over thousands of rows and its inverse
+    // amplifies their rounding: each chunk's fp32 sum is added in float64.
+    using f64x16 = __attribute__((ext_vector_type(16))) double;
+    f64x16 sum[MODE == kUpperReversed ? MT : 1][MODE == kUpperReversed ? NT : 1] = {};
     float4 va[BM / 64], vb[BN / 64];
     sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, 0, g.vecA);
     sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, 0, g.vecB);
@@ -172,6 +176,16 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
                     for (int y = 0; y < NT; ++y)
                         acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[x][e], fb[y][e], acc[x][y], 0, 0, 0);
         }
+        if constexpr (MODE == kUpperReversed) {
+#pragma unroll
+            for (int x = 0; x < MT; ++x)
+#pragma unroll
+                for (int y = 0; y < NT; ++y) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) sum[x][y][r] += (double)acc[x][y][r];
+                    acc[x][y] = f32x16{};
+                }
+        }
         if (more) {
             sgemm_stash<TA, BM>(As[buf ^ 1], va);
             sgemm_stash<TB ^ 1, BN>(Bs[buf ^ 1], vb);
@@ -188,10 +202,10 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
             for (int r = 0; r < 16; ++r) {
                 const int i = bi + wi + 32 * x + (r & 3) + 8 * (r >> 2) + 4 * h, j = bj + wj + 32 * y + li;
                 if (i >= M || j >= N) continue;
-                const float v = g.alpha * acc[x][y][r];
-                if (MODE == kUpperReversed) {
-                    if (j >= i) g.c[(size_t)(M - 1 - i) * g.ldc + (N - 1 - j)] = v;
+                if constexpr (MODE == kUpperReversed) {
+                    if (j >= i) g.c[(size_t)(M - 1 - i) * g.ldc + (N - 1 - j)] = (float)sum[x][y][r];
                 } else {
+                    const float v = g.alpha * acc[x][y][r];
                     float *p = g.c + (size_t)i * g.ldc + j;
                     *p = g.accumulate ? *p + v : v;
                 }
@@ -251,102 +265,198 @@ __global__ __launch_bounds__(1024) void gptq_damp_kernel(float *a, int n, uint8_
 // update. X's rows come from the sums over all rows above them, as in a
 // substitution, so L X = I holds to fp32 rounding of |L||X| (products of
 // inverted blocks, X21 = -X22 (L21 X11), have no such bound). K = 4096 from
-// 4096 rows: 53.5 -> 5.56 ms (separate launches for the block, the panel's
+// 4096 rows: 53.5 -> 2.91 ms (separate launches for the block, the panel's
 // substitution and the update, then one thin product and a substitution per 64
 // rows of the inverse, took 84 + 207 + 21 + 357 + 137 us a panel).
 
 // The packed lower triangle of a 64 x 64 block: row r, column c <= r.
 __device__ __forceinline__ int packed(int r, int c) { return r * (r + 1) / 2 + c; }
 
-// Factors the b x b (b <= 64) diagonal block held in S (lower triangle) and
-// inverts the factor, with 256 threads: choleskyLower's inner loop
-// (gptq_linalg.go:73-93) with float64 sums and pivot roots, L rounded to
-// float32 as it is formed. L goes to l (row stride ld), L^-1 to x as float32
-// (row stride ld) and, unless inv is null (no panel follows), to inv as packed
-// float64 for the panel product. Thread
-// (i, q) holds columns 4k + q of row i of the block and of the inverse, which
-// starts as the identity and takes the same row operations. Each of the 64
-// steps costs a float64 root and reciprocal, one LDS exchange and one barrier:
-// a chain of 52 us, longer than the other blocks' update beside it.
-__device__ void chol_diag(const float (*S)[65], double (*col)[64], float (*Ls)[65], int b, float *l, float *x,
-                          long ld, double *inv, int *bad) {
-    const int i = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    double a[16], w[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int c = 4 * k + q;
-        // Past b the block continues as the identity.
-        a[k] = i < b ? (c <= i ? (double)S[i][c] : 0.0) : (c == i ? 1.0 : 0.0);
-        w[k] = c == i ? 1.0 : 0.0;
-    }
-    const auto lane_of = [](double v, int from) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, from);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), from);
-        return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-    };
-#pragma unroll
-    for (int k0 = 0; k0 < 16; ++k0)
-#pragma unroll 1
-        for (int jj = 0; jj < 4; ++jj) {
-            const int j = 4 * k0 + jj;
-            if (q == jj) {  // this wavefront holds column j
-                double d = lane_of(a[k0], j);
-                if (!(d > 0.0)) {
-                    if (i == 0 && j < b) *bad = 1;
-                    d = 1.0;
-                }
-                const double piv = sqrt(d);
-                const float v = i == j ? (float)piv : i > j ? (float)(a[k0] / piv) : 0.0f;
-                Ls[i][j] = v;
-                col[j & 1][i] = (double)v;
-            }
-            __syncthreads();
-            const double *cj = col[j & 1];
-            const double li = cj[i], ljj = 1.0 / cj[j];
-            // Rows past j lose L[i][j] times row j; row j of the inverse is scaled.
-            const double f = i > j ? li : 0.0;
-#pragma unroll
-            for (int k = k0; k < 16; ++k) a[k] -= f * cj[4 * k + q];
-#pragma unroll
-            for (int k = 0; k <= k0; ++k) {
-                const double xj = lane_of(w[k], j) * ljj;
-                w[k] = i == j ? xj : w[k] - f * xj;
-            }
-        }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int c = 4 * k + q;
-        if (i < b && c <= i) {
-            x[(size_t)i * ld + c] = (float)w[k];
-            if (inv) inv[packed(i, c)] = w[k];
-        }
-    }
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int r = e >> 6, c = e & 63;
-        if (r < b && c <= r) l[(size_t)r * ld + c] = Ls[r][c];
-    }
+using f64x4 = __attribute__((ext_vector_type(4))) double;
+
+// Lane N's value in each row of 16 lanes (DPP row_newbcast).
+template <int N>
+__device__ __forceinline__ double row_bcast(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, 0x150 + N, 0xF, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), 0x150 + N, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// The diagonal block's working storage: D's lower 16 x 16 blocks hold A, then
+// L; an upper block (c, r) holds block (r, c) of S, then of L^-1, transposed;
+// V the diagonal blocks of L^-1.
 struct DiagLds {
-    float S[64][65], Ls[64][65];
-    double col[2][64];
+    double D[64][66];
+    double V[4][16][18];
 };
 
-// The first diagonal block.
-__global__ __launch_bounds__(256) void chol_first_kernel(float *a, int n, float *x, double *inv, int *bad) {
-    __shared__ DiagLds d;
-    const int b = min(64, n);
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int r = e >> 6, c = e & 63;
-        d.S[r][c] = r < b && c <= r ? a[(size_t)r * n + c] : 0.0f;
+// a[c] -= li L[c][J] for c = C .. 15, l holding L[.][J] by lane.
+template <int J, int C>
+__device__ __forceinline__ void chol16_row(double (&a)[16], double l, double li) {
+    if constexpr (C < 16) {
+        a[C] = fma(-li, row_bcast<C>(l), a[C]);
+        // Kept here: sunk to their use, 15 columns of broadcasts spill.
+        asm volatile("" : "+v"(a[C]));
+        chol16_row<J, C + 1>(a, l, li);
     }
-    __syncthreads();
-    chol_diag(d.S, d.col, d.Ls, b, a, x, n, inv, bad);
 }
 
-using f64x4 = __attribute__((ext_vector_type(4))) double;
+template <int J>
+__device__ __forceinline__ void chol16_steps(double (&a)[16], double (&w)[4], int i, bool &fail) {
+    if constexpr (J < 16) {
+        double d = row_bcast<J>(a[J]);
+        const bool positive = d > 0.0;
+        fail = fail || !positive;
+        d = positive ? d : 1.0;
+        // sqrt(d) and its reciprocal from the hardware's estimate, two Goldschmidt steps.
+        double r = __builtin_amdgcn_rsq(d), piv = d * r, hr = 0.5 * r;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const double e = fma(-piv, hr, 0.5);
+            piv = fma(piv, e, piv);
+            hr = fma(hr, e, hr);
+        }
+        r = 2.0 * hr;
+        // choleskyLower's column (gptq_linalg.go:73-93), stored as float32.
+        const double l = (double)(i == J ? (float)piv : (float)(a[J] * r));
+        a[J] = l;
+        const double li = i > J ? l : 0.0;
+        chol16_row<J, J + 1>(a, l, li);
+        // The reciprocal of the stored pivot; row J of the inverse is final.
+        const double ljj = row_bcast<J>(l);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) r = fma(r, fma(-ljj, r, 1.0), r);
+        const double lr = li * r;
+#pragma unroll
+        for (int k = 0; k <= J / 4; ++k) {
+            const double t = row_bcast<J>(w[k]);
+            w[k] = i == J ? t * r : fma(-lr, t, w[k]);
+            asm volatile("" : "+v"(w[k]));
+        }
+        chol16_steps<J + 1>(a, w, i, fail);
+    }
+}
+
+// Factors D's 16 x 16 diagonal block kb and inverts the factor into V, on one
+// wavefront: lane l holds row l % 16 of the block (a copy in each row of 16
+// lanes) and columns 4k + l / 16 of that row of the inverse.
+__device__ __forceinline__ void chol16(DiagLds &s, int kb, int *bad) {
+    const int i = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4, o = 16 * kb;
+    double a[16], w[4];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) a[c] = s.D[o + i][o + c];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = 4 * k + g == i ? 1.0 : 0.0;
+    bool fail = false;
+    chol16_steps<0>(a, w, i, fail);
+    if (fail && threadIdx.x == 0) *bad = 1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s.V[kb][i][4 * k + g] = w[k];
+    if (g == 0) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) s.D[o + i][o + c] = a[c];
+    }
+}
+
+// acc +- the 16 x 16 x 16 product of A (rows [i][p] at pa, stride lda) and B
+// ([j][p] at pb). Result register r of lane l: row 4 r + l / 16, column l % 16.
+__device__ __forceinline__ f64x4 mma16(const double *pa, int lda, const double *pb, int ldb, f64x4 acc) {
+    const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int p = 0; p < 16; p += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[li * lda + p + lk], pb[li * ldb + p + lk], acc, 0, 0, 0);
+    return acc;
+}
+
+// Factors the b x b (b <= 64) diagonal block whose lower triangle D holds
+// (identity past b) and inverts the factor, with 256 threads, float64
+// throughout, L rounded to float32 as it is formed. L goes to l (row stride
+// ld), L^-1 to x as float32 (row stride ld) and, unless inv is null (no panel
+// follows), to inv as packed float64 for the panel product. 16 columns at a
+// time: wavefront 0 factors the 16 x 16 block in registers while the others
+// finish the previous columns' products on v_mfma_f64_16x16x4_f64. A chain of
+// 64 columns, each a float64 root and its broadcasts: 16.5 us with the launch
+// (52 us as one loop over LDS with a root, two divisions and a barrier a column).
+__device__ __forceinline__ void chol_diag(DiagLds &s, int b, float *l, float *x, long ld, double *inv, int *bad) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+    for (int kb = 0; kb < 4; ++kb) {
+        // The products of block column kb - 1: tile 0 is the diagonal block that
+        // wavefront 0 goes on to factor.
+        const int q = kb - 1, trail = kb ? (4 - kb) * (5 - kb) / 2 : 0, tiles = kb ? trail + (4 - kb) * kb : 0;
+        for (int t = wave; t < tiles; t += wave ? 3 : 1000) {
+            int rb, cb;
+            if (t < trail) {
+                int row = 0, rest = t;
+                while (rest > row) rest -= ++row;
+                rb = kb + row;
+                cb = kb + rest;
+            } else {
+                rb = kb + (t - trail) / kb;
+                cb = (t - trail) % kb;
+            }
+            const bool minus = t < trail, fresh = !minus && cb == q;
+            f64x4 acc = {};
+            if (fresh) {
+#pragma unroll
+                for (int p = 0; p < 16; p += 4)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(s.D[16 * rb + li][16 * q + p + lk], s.V[q][p + lk][li],
+                                                               acc, 0, 0, 0);
+            } else {
+                acc = mma16(&s.D[16 * rb][16 * q], 66, &s.D[16 * cb][16 * q], 66, acc);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double *d = minus ? &s.D[16 * rb + 4 * r + lk][16 * cb + li] : &s.D[16 * cb + li][16 * rb + 4 * r + lk];
+                *d = minus ? *d - acc[r] : fresh ? acc[r] : *d + acc[r];
+            }
+        }
+        if (wave == 0) chol16(s, kb, bad);
+        __syncthreads();
+        // Column kb of L below its diagonal block, row kb of L^-1 beside its own.
+        if (wave < 3) {
+            const int t = wave < kb ? wave : wave + 1;
+            if (t > kb) {
+                const f64x4 acc = mma16(&s.D[16 * t][16 * kb], 66, &s.V[kb][0][0], 18, f64x4{});
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s.D[16 * t + 4 * r + lk][16 * kb + li] = (double)(float)acc[r];
+            } else {
+                const f64x4 acc = mma16(&s.V[kb][0][0], 18, &s.D[16 * t][16 * kb], 66, f64x4{});
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s.D[16 * t + li][16 * kb + 4 * r + lk] = -acc[r];
+            }
+        }
+        __syncthreads();
+    }
+    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
+        const int r = e >> 6, c = e & 63;
+        if (r >= b || c > r) continue;
+        const double v = (r >> 4) == (c >> 4) ? s.V[r >> 4][r & 15][c & 15] : s.D[c][r];
+        l[(size_t)r * ld + c] = (float)s.D[r][c];
+        x[(size_t)r * ld + c] = (float)v;
+        if (inv) inv[packed(r, c)] = v;
+    }
+}
+
+// The first diagonal block.
+__global__ __launch_bounds__(256, 3) void chol_first_kernel(float *a, int n, float *x, double *inv, int *bad) {
+    __shared__ DiagLds d;
+    const int b = min(64, n);
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = (int)threadIdx.x + 256 * u;
+        v[u] = a[(size_t)min(e >> 6, b - 1) * n + min(e & 63, b - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = (int)threadIdx.x + 256 * u, r = e >> 6, c = e & 63;
+        d.D[r][c] = r < b && c <= r ? (double)v[u] : r == c ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    chol_diag(d, b, a, x, n, inv, bad);
+}
 
 // The step at j0, on v_mfma_f64_16x16x4_f64. Blocks below `below`: 32 panel
 // rows each, L21 = A21 L11^-T (gptq_linalg.go:97-110). The others: 32 columns
@@ -357,32 +467,47 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(float *a, float *x, int
     __shared__ float Ar[64][36];   // the panel's 32 rows as [p][row], or S's 32 columns as [p][column]
     const bool rows = (int)blockIdx.x < below;
     const int i0 = rows ? j0 + 64 + (int)blockIdx.x * 32 : ((int)blockIdx.x - below) * 32;
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int r = e >> 6, c = e & 63;
-        Li[r][c] = c <= r ? inv[packed(r, c)] : 0.0;
+    // Every load unconditional (clamped; what lies past an edge feeds only
+    // results that are not stored): a guarded load is waited for on its own.
+    double lv[16];
+    float av[8];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = (int)threadIdx.x + 256 * u, r = e >> 6, c = e & 63;
+        lv[u] = inv[packed(r, min(c, r))];
     }
-    for (int e = threadIdx.x; e < 32 * 64; e += 256) {
-        if (rows) {
-            const int r = e >> 6, c = e & 63;
-            Ar[c][r] = i0 + r < n ? a[(size_t)(i0 + r) * n + j0 + c] : 0.0f;
-        } else {
-            const int r = e >> 5, c = e & 31;
-            Ar[r][c] = j0 + r < n ? x[(size_t)(j0 + r) * n + i0 + c] : 0.0f;
-        }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int e = (int)threadIdx.x + 256 * u;
+        av[u] = rows ? a[(size_t)min(i0 + (e >> 6), n - 1) * n + j0 + (e & 63)]
+                     : x[(size_t)min(j0 + (e >> 5), n - 1) * n + i0 + (e & 31)];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = (int)threadIdx.x + 256 * u, r = e >> 6, c = e & 63;
+        Li[r][c] = c <= r ? lv[u] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int e = (int)threadIdx.x + 256 * u;
+        if (rows) Ar[e & 63][e >> 6] = av[u];
+        else Ar[e >> 5][e & 31] = av[u];
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
     // Wavefront w: L11^-1's rows 16w .. 16w+15, which need p <= 16w + 15.
     f64x4 acc[2] = {};
-    for (int p = 0; p < 16 * (wave + 1); p += 4) {
-        const double lv = Li[16 * wave + li][p + lk];
+    for (int p0 = 0; p0 <= 16 * wave; p0 += 16)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const double v = (double)Ar[p + lk][16 * t + li];
-            acc[t] = rows ? __builtin_amdgcn_mfma_f64_16x16x4f64(v, lv, acc[t], 0, 0, 0)
-                          : __builtin_amdgcn_mfma_f64_16x16x4f64(lv, v, acc[t], 0, 0, 0);
+        for (int p = p0; p < p0 + 16; p += 4) {
+            const double lr = Li[16 * wave + li][p + lk];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const double v = (double)Ar[p + lk][16 * t + li];
+                acc[t] = rows ? __builtin_amdgcn_mfma_f64_16x16x4f64(v, lr, acc[t], 0, 0, 0)
+                              : __builtin_amdgcn_mfma_f64_16x16x4f64(lr, v, acc[t], 0, 0, 0);
+            }
         }
-    }
     // Result register r of lane l: row 4 r + l / 16, column l % 16.
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -403,7 +528,7 @@ __global__ __launch_bounds__(256) void chol_panel_kernel(float *a, float *x, int
 // lower triangle; block 0 then factors and inverts the diagonal block it has
 // just updated, the next step's. The others: S += L21 X[j0 .. j0+63], the
 // columns of the diagonal block for the first time.
-__global__ __launch_bounds__(256) void chol_update_kernel(float *a, int n, int j0, int tri, float *x, double *inv,
+__global__ __launch_bounds__(256, 3) void chol_update_kernel(float *a, int n, int j0, int tri, float *x, double *inv,
                                                           int *bad, int vec) {
     __shared__ union {
         struct {
@@ -426,27 +551,37 @@ __global__ __launch_bounds__(256) void chol_update_kernel(float *a, int n, int j
     const bool fresh = !trailing && bj == j0;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, h = lane >> 5;
     const int wi = (wave >> 1) * 32, wj = (wave & 1) * 32;
+    // Every load unconditional, rows and columns past the edge clamped (they
+    // feed only results that are not stored), the tile's own values among them.
+    float4 va[4], vb[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int idx = (int)threadIdx.x + 256 * e, r = idx >> 4, q = (idx & 15) * 4;
-        float4 va = make_float4(0, 0, 0, 0), vb = va;
-        const float *pa = a + (size_t)(bi + r) * n + j0 + q;
-        if (bi + r < n) va = vec ? *(const float4 *)pa : make_float4(pa[0], pa[1], pa[2], pa[3]);
+        const float *pa = a + (size_t)min(bi + r, n - 1) * n + j0 + q;
         // L21's rows [j][p], or the inverse's rows [p][j] (its diagonal block is lower).
-        const float *pb = trailing ? a + (size_t)(bj + r) * n + j0 + q : x + (size_t)(j0 + r) * n + bj + q;
-        if (!trailing || bj + r < n) vb = vec ? *(const float4 *)pb : make_float4(pb[0], pb[1], pb[2], pb[3]);
-        if (fresh)
-            vb = make_float4(q <= r ? vb.x : 0.0f, q + 1 <= r ? vb.y : 0.0f, q + 2 <= r ? vb.z : 0.0f,
-                             q + 3 <= r ? vb.w : 0.0f);
-        *(float4 *)&sh.p.A[r][q] = va;
-        *(float4 *)&sh.p.B[r][q] = vb;
+        const float *pb = trailing ? a + (size_t)min(bj + r, n - 1) * n + j0 + q : x + (size_t)(j0 + r) * n + bj + q;
+        if (vec) {
+            va[e] = *(const float4 *)pa;
+            vb[e] = *(const float4 *)pb;
+        } else {
+            va[e] = make_float4(pa[0], pa[1], pa[2], pa[3]);
+            vb[e] = make_float4(pb[0], pb[1], pb[2], pb[3]);
+        }
     }
-    // The tile's own values, in flight during the product.
     float own[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int i = bi + wi + (r & 3) + 8 * (r >> 2) + 4 * h, j = bj + wj + li;
-        own[r] = i < n && j <= i && !fresh ? c[(size_t)i * n + j] : 0.0f;
+        own[r] = c[(size_t)min(i, n - 1) * n + min(j, n - 1)];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int idx = (int)threadIdx.x + 256 * e, r = idx >> 4, q = (idx & 15) * 4;
+        if (fresh)
+            vb[e] = make_float4(q <= r ? vb[e].x : 0.0f, q + 1 <= r ? vb[e].y : 0.0f, q + 2 <= r ? vb[e].z : 0.0f,
+                                q + 3 <= r ? vb[e].w : 0.0f);
+        *(float4 *)&sh.p.A[r][q] = va[e];
+        *(float4 *)&sh.p.B[r][q] = vb[e];
     }
     __syncthreads();
     f32x16 acc = {};
@@ -470,14 +605,14 @@ __global__ __launch_bounds__(256) void chol_update_kernel(float *a, int n, int j
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int lr = wi + (r & 3) + 8 * (r >> 2) + 4 * h, lc = wj + li;
-        const float v = trailing ? own[r] - acc[r] : own[r] + acc[r];
-        if (diag) sh.d.S[lr][lc] = v;
+        const float v = trailing ? own[r] - acc[r] : fresh ? acc[r] : own[r] + acc[r];
+        // Past the matrix's edge the diagonal block continues as the identity.
+        if (diag) sh.d.D[lr][lc] = bi + lr < n ? (double)v : lr == lc ? 1.0 : 0.0;
         else if (bi + lr < n && bj + lc <= bi + lr) c[(size_t)(bi + lr) * n + bj + lc] = v;
     }
     if (!diag) return;
     __syncthreads();
-    chol_diag(sh.d.S, sh.d.col, sh.d.Ls, min(64, n - j1), a + (size_t)j1 * n + j1, x + (size_t)j1 * n + j1, n, inv,
-              bad);
+    chol_diag(sh.d, min(64, n - j1), a + (size_t)j1 * n + j1, x + (size_t)j1 * n + j1, n, inv, bad);
 }
 
 // U[r][c] = X[n-1-r][n-1-c] for c >= r, else 0 (gptq_linalg.go:208-221).
