@@ -9,16 +9,18 @@
 //   * vec_prep_blocks_kernel scales each 32-value block of each vector by an
 //     exact power of two 2^e (its max into [2^14, 2^15)) and splits it into
 //     FP16 hi + lo parts (x*2^e = hi + lo + r, |r| <= 2^-22 |x*2^e|), laid out
-//     as MFMA A fragments: rows 2v (hi) and 2v+1 (lo) of tile v/8;
-//   * gemv_vec2_kernel widens each 32-value block of 16 weight rows to FP16
-//     (int8 and 4-bit codes are exact in FP16), runs one
-//     v_mfma_f32_16x16x32_f16 per 16 A rows (products exact in fp32), and
-//     folds the block result into fp32 accumulators with the weight block
-//     scale and the activation block's 2^-e: acc = fma(d*2^-e, C, acc), the
-//     per-block scaling of the qwen3lm kernels;
-//   * K is split over wavefronts; partial sums meet in a fixed LDS tree;
+//     as MFMA A fragments;
+//   * vecs_kernel widens each 32-value block of 16 weight rows to FP16 (int8
+//     and 4-bit codes are exact in FP16), runs v_mfma_f32_16x16x32_f16 on it
+//     (products exact in fp32), and folds the block result into fp32
+//     accumulators with the weight block scale and the activation block's
+//     2^-e: acc = fma(d*2^-e, C, acc), the per-block scaling of the qwen3lm
+//     kernels;
+//   * K is split over wavefronts; partial sums meet in LDS in slice order;
 //     y[v][n] = acc_hi + acc_lo (Q8: times the row scale; PRO_NORM: times
 //     1/sqrt(mean(x^2) + eps) from the prep pass's block sums of squares).
+// 8-bit formats with up to 16 vectors and K a multiple of 512 take
+// vech_kernel (one scale per vector).
 // VALU work per weight does not grow with V.
 #include "common.h"
 
@@ -70,49 +72,59 @@ __host__ __device__ inline size_t vec_a_offset(int t, int kb, int KB, int lane) 
 }
 
 // ---- multi-vector GEMV with per-block activation scales ----------------------
-// vec_prep_blocks_kernel: one thread per (vector v, 32-value block kb). The
-// block's values are scaled by 2^e (its max into [2^14, 2^15)) and split into
-// FP16 hi + lo, written as the MFMA A fragments of rows 2v (hi) and 2v+1 (lo)
-// of tile v/8; inv[v][kb] = 2^-e and ssq[v][kb] = the block's sum of squares
-// (for PRO_NORM). Every thread is independent, so the pass takes one short
-// launch for any vector count.
+// The A tiles of V vectors: up to 8 vectors, one tile with hi and lo of vector
+// v in rows 2v and 2v + 1; up to 16, a hi tile and a lo tile with vector v in
+// row v (PAIR, half the result registers); more, the first kind, 8 vectors a
+// tile.
+__host__ __device__ inline bool vec_pair(int V) { return V > 8 && V <= 16; }
+
+// vec_prep_blocks_kernel: four threads per (vector v, 32-value block kb), 8
+// values each. The block's values are scaled by 2^e (its max into [2^14,
+// 2^15)) and split into FP16 hi + lo, written as the MFMA A fragments;
+// inv[v][kb] = 2^-e and ssq[v][kb] = the block's sum of squares (for
+// PRO_NORM). Every block is independent, so the pass takes one short launch
+// for any vector count.
 __global__ __launch_bounds__(256) void vec_prep_blocks_kernel(const float *__restrict__ x, long stride, int V, int KB,
                                                               _Float16 *__restrict__ A, float *__restrict__ inv,
                                                               float *__restrict__ ssq) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= V * KB) return;
-    const int v = idx / KB, kb = idx - v * KB;
-    const float4 *xp = (const float4 *)(x + (size_t)v * stride + (size_t)kb * 32);
-    float xs[32];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float4 q = xp[i];
-        xs[4 * i] = q.x, xs[4 * i + 1] = q.y, xs[4 * i + 2] = q.z, xs[4 * i + 3] = q.w;
-    }
+    const long t4 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int gq = (int)(t4 & 3);
+    const long idx = min(t4 >> 2, (long)V * KB - 1);  // the last block's extra threads repeat its work
+    const int v = (int)(idx / KB), kb = (int)(idx - (long)v * KB);
+    const float4 *xp = (const float4 *)(x + (size_t)v * stride + (size_t)kb * 32 + gq * 8);
+    const float4 q0 = xp[0], q1 = xp[1];
+    const float xs[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
     float mx = 0.0f, ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < 8; ++i) {
         mx = fmaxf(mx, fabsf(xs[i]));
         ss += xs[i] * xs[i];
     }
+    // The block's other three quarters sit in the neighbouring lanes.
+#pragma unroll
+    for (int off = 1; off < 4; off <<= 1) {
+        mx = fmaxf(mx, __shfl_xor(mx, off));
+        ss += __shfl_xor(ss, off);
+    }
     const int e = pow2_exponent(mx);
     const float sc = pow2f(e);
-    const int t = v >> 3, rHi = (2 * v) & 15, rLo = rHi + 1;
+    f16x8 hi, lo;
 #pragma unroll
-    for (int gq = 0; gq < 4; ++gq) {
-        f16x8 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float y = xs[gq * 8 + i] * sc;  // exact: a power-of-two scaling
-            const _Float16 h = (_Float16)y;
-            hi[i] = h;
-            lo[i] = (_Float16)(y - (float)h);
-        }
-        *(f16x8 *)(A + vec_a_offset(t, kb, KB, gq * 16 + rHi)) = hi;
-        *(f16x8 *)(A + vec_a_offset(t, kb, KB, gq * 16 + rLo)) = lo;
+    for (int i = 0; i < 8; ++i) {
+        const float y = xs[i] * sc;  // exact: a power-of-two scaling
+        const _Float16 h = (_Float16)y;
+        hi[i] = h;
+        lo[i] = (_Float16)(y - (float)h);
     }
-    inv[idx] = pow2f(-e);
-    ssq[idx] = ss;
+    const bool pair = vec_pair(V);
+    const int th = pair ? 0 : v >> 3, tl = pair ? 1 : th;
+    const int rh = pair ? v : (2 * v) & 15, rl = pair ? v : rh + 1;
+    *(f16x8 *)(A + vec_a_offset(th, kb, KB, gq * 16 + rh)) = hi;
+    *(f16x8 *)(A + vec_a_offset(tl, kb, KB, gq * 16 + rl)) = lo;
+    if (gq == 0) {
+        inv[idx] = pow2f(-e);
+        ssq[idx] = ss;
+    }
 }
 
 struct Vec2Args {
@@ -128,159 +140,265 @@ struct Vec2Args {
     float *part;  // K-split stationary path: [parts][V][N] partial sums
 };
 
-// Multi-vector GEMV over prepared A fragments: each wavefront applies its A
-// fragments to RT tiles of 16 weight rows, U blocks at a time. All U*RT*MT
-// MFMAs of a step are issued before their results are scaled and summed
-// (acc += d * 2^-e_v * C), which keeps the MFMA latency off the critical path.
-// VALU work per weight is the code conversion (v_perm + packed FP16
-// subtract). K is split over the SK wavefronts of the block; partial sums meet
-// in a fixed LDS tree, and PRO_NORM's sum of squares is read from the prep
-// pass's block sums in block order.
-template <int FMT, int MT, int SK, int RT, int U, int EPI, bool NORM>
-__global__ __launch_bounds__(64 * SK) void gemv_vec2_kernel(const Vec2Args a) {
-    static_assert((SK & (SK - 1)) == 0, "SK is a power of two");
-    __shared__ f32x4 red[(SK > 1 ? SK / 2 : 1) * RT * MT * 64];
-    const int lane = threadIdx.x & 63;
-    const int ks = threadIdx.x >> 6;
-    const int g = lane >> 4, m = lane & 15;
-    const int n0 = blockIdx.x * (RT * 16);
-    const int KB = a.KB;
-    const int per = ((KB + SK - 1) / SK + U - 1) / U * U;  // whole U-groups per wavefront
-    const int kb0 = ks * per, kb1 = min(KB, kb0 + per);
-    const int8_t *wrow[RT];
-    const uint8_t *srow[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int row = min(n0 + rt * 16 + m, a.N - 1);
-        wrow[rt] = FMT == GPHQ_FMT_Q4 ? (const int8_t *)a.codes + (size_t)row * (a.K >> 1) + (g & 1) * 8
-                                      : (const int8_t *)a.codes + (size_t)row * a.K + g * 8;
-        srow[rt] = (const uint8_t *)a.scales + (size_t)row * KB * (FMT == GPHQ_FMT_Q8B_F32 ? 4 : 2);
-    }
-    // The lane's C rows 4g..4g+3 of tile t are vectors t*8 + 2g (hi, lo) and t*8 + 2g + 1.
-    const float *invp[MT][2];
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) invp[t][p] = a.inv + (size_t)min(t * 8 + 2 * g + p, a.V - 1) * KB;
-    f32x4 acc[RT][MT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+// How a vecs_kernel launch cuts K: `parts` passes over the block's row tiles,
+// each over SK wavefronts' slices of nb 32-value blocks.
+struct VecsShape {
+    int iters, SK, nb, parts;
+    int svec;  // block scales load as one aligned vector per lane
+};
 
-    for (int kbs = kb0; kbs < kb1; kbs += U) {
-        f16x8 av[U][MT];
-        u32x2 w[U][RT];
-        float d[U][RT], iv[U][MT][2];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int kb = min(kbs + u, KB - 1);
-            const bool ok = kbs + u < kb1;
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                av[u][t] = *(const f16x8 *)(a.A + vec_a_offset(t, kb, KB, lane));
-                iv[u][t][0] = ok ? invp[t][0][kb] : 0.0f;
-                iv[u][t][1] = ok ? invp[t][1][kb] : 0.0f;
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                w[u][rt] = *(const u32x2 *)(wrow[rt] + (size_t)kb * (FMT == GPHQ_FMT_Q4 ? 16 : 32));
-                if constexpr (FMT == GPHQ_FMT_Q8B || FMT == GPHQ_FMT_Q4)
-                    d[u][rt] = half_bits_to_float(((const uint16_t *)srow[rt])[kb]);
-                else if constexpr (FMT == GPHQ_FMT_Q8B_F32)
-                    d[u][rt] = ((const float *)srow[rt])[kb];
-                else
-                    d[u][rt] = 1.0f;
-            }
-        }
-        f32x4 c[U][RT][MT];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const f16x8 b = FMT == GPHQ_FMT_Q4 ? u4x8_to_f16(w[u][rt], (g >> 1) * 4) : i8x8_to_f16(w[u][rt]);
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    c[u][rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[u][t], b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const float d0 = d[u][rt] * iv[u][t][0], d1 = d[u][rt] * iv[u][t][1];
-                    acc[rt][t][0] = fmaf(d0, c[u][rt][t][0], acc[rt][t][0]);
-                    acc[rt][t][1] = fmaf(d0, c[u][rt][t][1], acc[rt][t][1]);
-                    acc[rt][t][2] = fmaf(d1, c[u][rt][t][2], acc[rt][t][2]);
-                    acc[rt][t][3] = fmaf(d1, c[u][rt][t][3], acc[rt][t][3]);
-                }
+// NB: 32-value blocks per slice, at most (their A fragments stay in registers).
+template <int FMT, int T, bool PAIR, int NB>
+struct VecsTraits {
+    static constexpr bool Q4 = FMT == GPHQ_FMT_Q4;
+    // Wavefronts of a block, at most: what the registers leave per SIMD (4, 3 or 2).
+    static constexpr int kMaxSK = !PAIR && T == 1 ? 16 : (PAIR ? 2 : T) * NB <= 16 ? 12 : 8;
+    static constexpr int WB = Q4 ? 16 : 32;                    // code bytes per block and row
+    static constexpr int STEPS = NB * WB / 128;                // 128-byte lines per row and slice
+    static constexpr int SB = FMT == GPHQ_FMT_Q8 ? 0 : FMT == GPHQ_FMT_Q8B_F32 ? 4 : 2;  // scale bytes per block
+    static constexpr int VC = PAIR ? 16 : 8 * T;               // vectors the tiles hold
+    static constexpr int CH = T > 2 ? 2 : 4;                   // tiles whose slice sums are reduced together
+    static constexpr int kStage = STEPS * 128 * 16, kScale = 16 * NB * SB, kInv = NB * VC * 4;
+    static constexpr int kWave = kStage + kScale + kInv;       // LDS bytes per wavefront
+    static constexpr int ch(int SK) { return SK < CH ? SK : CH; }
+    static int lds(int SK, int parts, int iters) {
+        return SK * kWave + (SK > 1 ? ch(SK) * SK * T * 1024 : 0) + (parts > 1 ? iters * T * 1024 : 0) +
+               (VC + 3) / 4 * 16;
     }
-#pragma unroll
-    for (int half = SK / 2; half >= 1; half >>= 1) {
-        if (ks >= half && ks < 2 * half) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int t = 0; t < MT; ++t) red[(((ks - half) * RT + rt) * MT + t) * 64 + lane] = acc[rt][t];
-        }
-        __syncthreads();
-        if (ks < half) {
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int t = 0; t < MT; ++t) acc[rt][t] += red[((ks * RT + rt) * MT + t) * 64 + lane];
-        }
-        __syncthreads();
-    }
-    if (ks != 0) return;
-    float nf[MT][2];
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) nf[t][p] = 1.0f;
+};
+
+// Multi-vector GEMV over prepared A fragments, any K a multiple of 32. What
+// bounds it is the weight stream together with the A fragments every CU reads
+// from L2 (V = 8, K = 4096: 128 KB beside 225 KB of 4-bit weights for 24576
+// rows), and for 4-bit codes the VALU work of widening them (12 instructions
+// per 16 x 32 codes). So each wavefront keeps its K slice's A fragments in
+// registers and walks 16-row tiles over a persistent grid; weights load as
+// 8 rows x 128 bytes per instruction (whole lines: 8 bytes per lane straight
+// into operands touch 16 lines per instruction and were address-bound) and
+// turn into B fragments through the wavefront's LDS, the next tile's loads in
+// flight meanwhile. Slices meet in LDS, a few tiles at a time. K past one
+// pass's slices takes further passes over the same tiles, whose sums wait in
+// LDS. 8 vectors, Q4, K = 4096, N = 24576: 65.4 -> 20.7
+// us with its preparation; 32 vectors 101.8 -> 44.8, 8 vectors at K = 12288, N =
+// 4096 35.3 -> 18.2.
+template <int FMT, int T, bool PAIR, int NB, int EPI, bool NORM>
+__global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void vecs_kernel(const Vec2Args a,
+                                                                                             const VecsShape sh) {
+    using X = VecsTraits<FMT, T, PAIR, NB>;
+    constexpr bool Q4 = X::Q4;
+    constexpr int WB = X::WB, STEPS = X::STEPS, SB = X::SB, VC = X::VC;
+    constexpr int AT = PAIR ? 2 : T;     // A tiles
+    constexpr int NI = PAIR ? 4 : 2;     // vectors of one result tile in a lane
+    constexpr int QB = NB / 4;           // scales per lane and tile
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int lane = threadIdx.x & 63;
+    const int ks = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int g = lane >> 4, m = lane & 15;
+    const int KB = a.KB, SK = sh.SK, nb = sh.nb, iters = sh.iters, CH = X::ch(SK);
+    u32x4 *const st = (u32x4 *)(smem + ks * X::kWave);
+    uint8_t *const ssc = smem + ks * X::kWave + X::kStage;
+    float *const siv = (float *)(ssc + X::kScale);
+    f32x4 *const part = (f32x4 *)(smem + SK * X::kWave);                      // [slot][slice][T][lane]
+    f32x4 *const held = part + (SK > 1 ? CH * SK * T * 64 : 0);               // [iteration][T][lane]
+    float *const nf = (float *)(held + (sh.parts > 1 ? iters * T * 64 : 0));  // [VC]
+    const int tiles = (a.N + 15) / 16;
+    const int rowBytes = KB * WB;
     if constexpr (NORM) {
-        // Each vector's block sums of squares, added by the whole wavefront in
-        // a fixed order; lane group g keeps vectors t*8 + 2g + {0, 1}.
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-#pragma unroll
-            for (int vv = 0; vv < 8; ++vv) {
-                const float *q = a.ssq + (size_t)min(t * 8 + vv, a.V - 1) * KB;
-                float part = 0.0f;
-                for (int kb = lane; kb < KB; kb += 64) part += q[kb];
-                const float tot = wave_sum(part);
-                if ((vv >> 1) == g) nf[t][vv & 1] = 1.0f / sqrtf(tot / (float)a.K + a.eps);
-            }
+        // Each vector's block sums of squares, added by one wavefront in a fixed order.
+        for (int v = ks; v < VC; v += SK) {
+            const float *q = a.ssq + (size_t)min(v, a.V - 1) * KB;
+            float s = 0.0f;
+            for (int kb = lane; kb < KB; kb += 64) s += q[kb];
+            s = wave_sum(s);
+            if (lane == 0) nf[v] = 1.0f / sqrtf(s / (float)a.K + a.eps);
         }
+        __syncthreads();
     }
+    u32x4 R[STEPS][2];
+    uint32_t S[SB ? QB : 1];
+    int kb0 = 0;
+    auto gload = [&](int t2) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int col = n0 + rt * 16 + m;
-        float rs = 1.0f;
-        if constexpr (FMT == GPHQ_FMT_Q8) rs = ((const float *)a.scales)[min(col, a.N - 1)];
+        for (int h2 = 0; h2 < 2; ++h2) {
+            const int mm = h2 * 8 + (lane >> 3);
+            const int c = (lane & 7) ^ (mm >> 1);
+            const int row = min(t2 * 16 + mm, a.N - 1);
+            const uint8_t *src = (const uint8_t *)a.codes + (size_t)row * rowBytes;
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
+            for (int s = 0; s < STEPS; ++s)  // past the row's end: its last chunk, times a zero activation
+                R[s][h2] = __builtin_nontemporal_load(
+                    (const u32x4 *)(src + min(kb0 * WB + s * 128 + c * 16, rowBytes - 16)));
+        }
+        if constexpr (SB > 0) {
+            // Lane l: row l / 4, QB blocks from (l % 4) QB.
+            const size_t base = (size_t)min(t2 * 16 + (lane >> 2), a.N - 1) * KB;
+            const int kq = kb0 + (lane & 3) * QB;
+            if (sh.svec) {
+                const uint8_t *p = (const uint8_t *)a.scales + (base + min(kq, KB - QB)) * SB;
+                if constexpr (QB * SB == 16) {
+                    const u32x4 w = *(const u32x4 *)p;
+                    S[0] = w.x, S[1] = w.y, S[2] = w.z, S[3] = w.w;
+                } else if constexpr (QB * SB == 8) {
+                    const u32x2 w = *(const u32x2 *)p;
+                    S[0] = w.x, S[1] = w.y;
+                } else {
+                    S[0] = *(const uint32_t *)p;
+                }
+            } else if constexpr (SB == 4) {
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const int v = t * 8 + 2 * g + p;
-                float val = (acc[rt][t][2 * p] + acc[rt][t][2 * p + 1]) * nf[t][p];
-                if constexpr (FMT == GPHQ_FMT_Q8) val *= rs;
-                if constexpr (EPI == VEC_SWIGLU) {
-                    const float up = __shfl_xor(val, 1);  // lane l^1 holds column col^1
-                    if (v < a.V && col < a.N && (col & 1) == 0)
-                        a.y[(size_t)v * a.ystride + (col >> 1)] = val / (1.0f + expf(-val)) * up;
-                } else if (v < a.V && col < a.N) {
-                    if constexpr (EPI == VEC_ADD)
-                        a.y[(size_t)v * a.ystride + col] += val;
-                    else
-                        a.y[(size_t)v * a.ystride + col] = val;
+                for (int i = 0; i < QB; ++i) S[i] = ((const uint32_t *)a.scales)[base + min(kq + i, KB - 1)];
+            } else {
+#pragma unroll
+                for (int i = 0; i < QB; i += 2) {
+                    const uint32_t lo = ((const uint16_t *)a.scales)[base + min(kq + i, KB - 1)];
+                    const uint32_t hi = ((const uint16_t *)a.scales)[base + min(kq + i + 1, KB - 1)];
+                    S[i / 2] = lo | hi << 16;
                 }
             }
+        }
+    };
+    auto lwrite = [&]() {
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+            for (int h2 = 0; h2 < 2; ++h2) st[s * 128 + h2 * 64 + lane] = R[s][h2];
+        if constexpr (SB > 0) {
+            uint8_t *d = ssc + ((lane >> 2) * NB + (lane & 3) * QB) * SB;
+#pragma unroll
+            for (int i = 0; i < QB * SB / 4; ++i) {
+                // Blocks past K scale by 0 (their codes are another block's).
+                const int kb = kb0 + (lane & 3) * QB + i * (4 / (SB ? SB : 1));
+                uint32_t w = S[i];
+                if (SB == 4) w = kb < KB ? w : 0;
+                else w = kb + 1 < KB ? w : kb < KB ? w & 0xFFFFu : 0;
+                __builtin_memcpy(d + 4 * i, &w, 4);
+            }
+        }
+    };
+    for (int part_i = 0; part_i < sh.parts; ++part_i) {
+        kb0 = min((part_i * SK + ks) * nb, KB);
+        const int mine = min(nb, KB - kb0);  // blocks of this slice (0: none left)
+        int tt = blockIdx.x;
+        gload(tt);
+        f16x8 av[NB][AT];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int t = 0; t < AT; ++t) {
+                if (b < mine) av[b][t] = *(const f16x8 *)(a.A + vec_a_offset(t, kb0 + b, KB, lane));
+                else av[b][t] = f16x8{};
+            }
+        for (int e = lane; e < NB * VC; e += 64) {
+            const int b = e / VC, v = e - b * VC;
+            const float iv = a.inv[(size_t)min(v, a.V - 1) * KB + min(kb0 + b, KB - 1)];
+            siv[e] = b < mine ? iv : 0.0f;
+        }
+        lwrite();
+        for (int it = 0; it < iters; ++it, tt += gridDim.x) {
+            const bool more = it + 1 < iters;
+            if (more) gload(tt + gridDim.x);  // past the last tile: its last row again
+            f32x4 acc[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            uint32_t sw[SB ? NB * SB / 4 : 1];  // the scales of this lane's row
+            if constexpr (SB > 0) __builtin_memcpy(sw, __builtin_assume_aligned(ssc + m * NB * SB, 8), NB * SB);
+#pragma unroll
+            for (int b4 = 0; b4 < NB; b4 += 4) {
+                if (b4 >= mine) break;
+#pragma unroll
+                for (int b = b4; b < b4 + 4; ++b) {
+                    constexpr int PER = 128 / WB;  // blocks per line
+                    const int c = Q4 ? b % PER : 2 * (b % PER) + (g >> 1);
+                    const u32x2 wv = *(const u32x2 *)((const uint32_t *)(st + (b / PER) * 128 + m * 8 + (c ^ (m >> 1))) +
+                                                      (g & 1) * 2);
+                    const f16x8 bf = Q4 ? u4x8_to_f16(wv, (g >> 1) * 4) : i8x8_to_f16(wv);
+                    float d = 1.0f;
+                    if constexpr (SB == 2) d = half_bits_to_float((uint16_t)((b & 1) ? sw[b / 2] >> 16 : sw[b / 2]));
+                    else if constexpr (SB == 4) d = __builtin_bit_cast(float, sw[b]);
+#pragma unroll
+                    for (int t = 0; t < T; ++t) {
+                        f32x4 cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[b][t], bf, f32x4{0.f, 0.f, 0.f, 0.f}, 0,
+                                                                          0, 0);
+                        if constexpr (PAIR) cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[b][1], bf, cc, 0, 0, 0);
+                        const float *iv = siv + b * VC + (PAIR ? 4 * g : 8 * t + 2 * g);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float f = iv[PAIR ? i : i >> 1];
+                            acc[t][i] = fmaf(SB ? d * f : f, cc[i], acc[t][i]);
+                        }
+                    }
+                }
+            }
+            if (more) lwrite();  // after this tile's LDS reads (LDS operations of a wavefront run in order)
+            // Result i of lane (g, m): row tile * 16 + m; PAIR: vector 4g + i; else
+            // hi and lo of vector 8t + 2g + i/2.
+            auto epilogue = [&](int ti, int tile, f32x4 (&r)[T]) {
+                if (part_i) {
+#pragma unroll
+                    for (int t = 0; t < T; ++t) r[t] = held[(ti * T + t) * 64 + lane] + r[t];
+                }
+                if (part_i + 1 < sh.parts) {
+#pragma unroll
+                    for (int t = 0; t < T; ++t) held[(ti * T + t) * 64 + lane] = r[t];
+                    return;
+                }
+                if (tile >= tiles) return;
+                const int col = tile * 16 + m;
+                float rs = 1.0f;
+                if constexpr (FMT == GPHQ_FMT_Q8) rs = ((const float *)a.scales)[min(col, a.N - 1)];
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+#pragma unroll
+                    for (int i = 0; i < NI; ++i) {
+                        const int v = PAIR ? 4 * g + i : 8 * t + 2 * g + i;
+                        float val = PAIR ? r[t][i] : r[t][2 * i] + r[t][2 * i + 1];
+                        if constexpr (NORM) val *= nf[v];
+                        if constexpr (FMT == GPHQ_FMT_Q8) val *= rs;
+                        if constexpr (EPI == VEC_SWIGLU) {
+                            const float up = __shfl_xor(val, 1);  // lane m^1 holds column col^1
+                            if (v < a.V && col < a.N && (col & 1) == 0)
+                                a.y[(size_t)v * a.ystride + (col >> 1)] = val / (1.0f + expf(-val)) * up;
+                        } else if (v < a.V && col < a.N) {
+                            if constexpr (EPI == VEC_ADD)
+                                a.y[(size_t)v * a.ystride + col] += val;
+                            else
+                                a.y[(size_t)v * a.ystride + col] = val;
+                        }
+                    }
+            };
+            if (SK == 1) {
+                epilogue(it, tt, acc);
+                continue;
+            }
+            const int slot = it % CH;
+#pragma unroll
+            for (int t = 0; t < T; ++t) part[((slot * SK + ks) * T + t) * 64 + lane] = acc[t];
+            if (slot != CH - 1 && it != iters - 1) continue;  // the same for every wavefront
+            __syncthreads();
+            if (ks <= slot) {
+                // Wavefront ks adds slot ks's slices in order: the tile slot - ks blocks back.
+                f32x4 r[T];
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const f32x4 *ps = part + (ks * SK * T + t) * 64 + lane;
+                    r[t] = ps[0];
+                    for (int k2 = 1; k2 < SK; ++k2) r[t] += ps[k2 * T * 64];
+                }
+                epilogue(it - (slot - ks), tt - (slot - ks) * (int)gridDim.x, r);
+            }
+            __syncthreads();
         }
     }
 }
 
+// K = 0: every product is an empty sum.
+template <int FMT>
+__global__ __launch_bounds__(256) void vec_empty_kernel(const Vec2Args a, bool store) {
+    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= (long)a.V * a.N || !store) return;
+    const int v = (int)(idx / a.N), col = (int)(idx - (long)v * a.N);
+    a.y[(size_t)v * a.ystride + col] = FMT == GPHQ_FMT_Q8 ? 0.0f * ((const float *)a.scales)[col] : 0.0f;
+}
 
 // ---- stationary activations: up to 16 vectors, 8-bit formats -------------------
 // For V <= 16 vectors and K a multiple of 512 up to 4096 the activations stay
@@ -683,39 +801,63 @@ size_t gemv_vec_workspace_bytes(int V, int K) {
     return (size_t)MT * KB * 1024 + 2 * (size_t)V * KB * 4 + 256;
 }
 
-// Tile shapes measured on MI355X (Qwen3-8B projections, 4 and 16 vectors):
-// up to 8192 rows, 16-row blocks of four K-slices with four blocks in flight;
-// taller matrices, 64-row blocks of eight K-slices with two in flight.
-template <int FMT, int MT, int EPI, bool NORM>
-static int launch_vec2(const Vec2Args &a, hipStream_t stream) {
-    if (a.N <= 8192) {
-        hipLaunchKernelGGL((gemv_vec2_kernel<FMT, MT, 4, 1, 4, EPI, NORM>), dim3((unsigned)((a.N + 15) / 16)),
-                           dim3(256), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((gemv_vec2_kernel<FMT, MT, 8, 4, 2, EPI, NORM>), dim3((unsigned)((a.N + 63) / 64)),
-                           dim3(512), 0, stream, a);
-    }
+// The slices of K: as few passes as hold KB blocks, each over as many
+// wavefronts as it has 128-byte lines. Every block reads all of its A
+// fragments, so few blocks of many slices move less than many blocks of few:
+// V = 12, K = 672, N = 9000, Q8B takes 12 us at two blocks of five slices a CU,
+// 10 us at one. Where the tiles' sums of a further pass would not fit in LDS,
+// more blocks walk fewer tiles.
+template <int FMT, int T, bool PAIR, int NB, int EPI, bool NORM>
+static int go_vecs(const Vec2Args &a, hipStream_t stream) {
+    using X = VecsTraits<FMT, T, PAIR, NB>;
+    constexpr int kMaxSK = X::kMaxSK, kLds = 160 << 10;
+    const int line = X::Q4 ? 8 : 4;  // blocks per 128-byte line
+    VecsShape sh{};
+    sh.parts = (a.KB + kMaxSK * NB - 1) / (kMaxSK * NB);
+    const int per = (a.KB + sh.parts - 1) / sh.parts;  // blocks of one pass
+    sh.SK = std::min(kMaxSK, (per + line - 1) / line);
+    sh.nb = std::min(NB, ((per + sh.SK - 1) / sh.SK + line - 1) / line * line);
+    sh.SK = (per + sh.nb - 1) / sh.nb;
+    sh.svec = X::SB && a.KB % 4 == 0 && (uintptr_t)a.scales % 16 == 0;
+    const int tiles = (a.N + 15) / 16;
+    int blocks = std::max(1, std::min(tiles, device_cus() * std::max(1, (T == 1 && !PAIR ? kMaxSK : 8) / sh.SK)));
+    sh.iters = (tiles + blocks - 1) / blocks;
+    const int room = (kLds - X::lds(sh.SK, 1, 0)) / (T * 1024);
+    if (sh.parts > 1 && sh.iters > room) sh.iters = room;
+    blocks = (tiles + sh.iters - 1) / sh.iters;
+    const int lds = X::lds(sh.SK, sh.parts, sh.iters);
+    if (lds > (64 << 10))
+        (void)hipFuncSetAttribute((const void *)vecs_kernel<FMT, T, PAIR, NB, EPI, NORM>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL((vecs_kernel<FMT, T, PAIR, NB, EPI, NORM>), dim3((unsigned)blocks), dim3(64 * sh.SK), lds, stream,
+                       a, sh);
     return launch_status();
 }
 
 template <int FMT, int EPI, bool NORM>
-static int launch_vec2_mt(const Vec2Args &a, hipStream_t stream) {
-    switch ((2 * a.V + 15) / 16) {
-    case 1: return launch_vec2<FMT, 1, EPI, NORM>(a, stream);
-    case 2: return launch_vec2<FMT, 2, EPI, NORM>(a, stream);
-    case 3: return launch_vec2<FMT, 3, EPI, NORM>(a, stream);
-    case 4: return launch_vec2<FMT, 4, EPI, NORM>(a, stream);
+static int launch_vecs_tiles(const Vec2Args &a, hipStream_t stream) {
+    if (vec_pair(a.V)) {
+        // Slices of 8 blocks leave three wavefronts per SIMD instead of two but
+        // hold K <= 3072 in one pass; a second pass costs more than they gain
+        // (V = 9, K = 1984, N = 17374, Q8: 19.3 us with 16 blocks, 15.9 with 8).
+        return a.KB <= 96 ? go_vecs<FMT, 1, true, 8, EPI, NORM>(a, stream)
+                          : go_vecs<FMT, 1, true, 16, EPI, NORM>(a, stream);
+    }
+    switch ((a.V + 7) / 8) {
+    case 1: return go_vecs<FMT, 1, false, 8, EPI, NORM>(a, stream);
+    case 3: return go_vecs<FMT, 3, false, 8, EPI, NORM>(a, stream);
+    case 4: return go_vecs<FMT, 4, false, 8, EPI, NORM>(a, stream);
     }
     return GPHQ_ERR_UNSUPPORTED;
 }
 
 template <int EPI, bool NORM>
-static int launch_vec2_fmt(int fmt, const Vec2Args &a, hipStream_t stream) {
+static int launch_vecs(int fmt, const Vec2Args &a, hipStream_t stream) {
     switch (fmt) {
-    case GPHQ_FMT_Q8: return launch_vec2_mt<GPHQ_FMT_Q8, EPI, NORM>(a, stream);
-    case GPHQ_FMT_Q8B: return launch_vec2_mt<GPHQ_FMT_Q8B, EPI, NORM>(a, stream);
-    case GPHQ_FMT_Q8B_F32: return launch_vec2_mt<GPHQ_FMT_Q8B_F32, EPI, NORM>(a, stream);
-    case GPHQ_FMT_Q4: return launch_vec2_mt<GPHQ_FMT_Q4, EPI, NORM>(a, stream);
+    case GPHQ_FMT_Q8: return launch_vecs_tiles<GPHQ_FMT_Q8, EPI, NORM>(a, stream);
+    case GPHQ_FMT_Q8B: return launch_vecs_tiles<GPHQ_FMT_Q8B, EPI, NORM>(a, stream);
+    case GPHQ_FMT_Q8B_F32: return launch_vecs_tiles<GPHQ_FMT_Q8B_F32, EPI, NORM>(a, stream);
+    case GPHQ_FMT_Q4: return launch_vecs_tiles<GPHQ_FMT_Q4, EPI, NORM>(a, stream);
     }
     return GPHQ_ERR_UNSUPPORTED;
 }
@@ -780,19 +922,23 @@ int gemv_vec_fused_launch(int fmt, int norm, int epi, const void *codes, const v
     _Float16 *A = (_Float16 *)work;
     float *inv = (float *)((char *)work + (size_t)MT * KB * 1024);
     float *ssq = inv + (size_t)V * KB;
-    // A rows past 2V in the last tile are never written; they only feed C
-    // rows that are never stored.
-    if (KB > 0) {
-        hipLaunchKernelGGL(vec_prep_blocks_kernel, dim3((unsigned)((V * KB + 255) / 256)), dim3(256), 0, stream, x,
-                           xstride, V, KB, A, inv, ssq);
-        GPHQ_TRY(launch_status());
-    }
     const Vec2Args a{codes, scales, A, inv, ssq, y, ystride, V, K, N, KB, eps};
-    if (epi == VEC_ADD) return norm ? launch_vec2_fmt<VEC_ADD, true>(fmt, a, stream)
-                                    : launch_vec2_fmt<VEC_ADD, false>(fmt, a, stream);
-    if (epi == VEC_SWIGLU) return norm ? launch_vec2_fmt<VEC_SWIGLU, true>(fmt, a, stream)
-                                       : launch_vec2_fmt<VEC_SWIGLU, false>(fmt, a, stream);
-    return norm ? launch_vec2_fmt<VEC_STORE, true>(fmt, a, stream) : launch_vec2_fmt<VEC_STORE, false>(fmt, a, stream);
+    if (KB == 0) {  // an empty sum: stored, or added as nothing
+        const dim3 grid((unsigned)(((long)V * N + 255) / 256));
+        if (fmt == GPHQ_FMT_Q8) hipLaunchKernelGGL(vec_empty_kernel<GPHQ_FMT_Q8>, grid, dim3(256), 0, stream, a, epi == VEC_STORE);
+        else hipLaunchKernelGGL(vec_empty_kernel<GPHQ_FMT_Q8B>, grid, dim3(256), 0, stream, a, epi == VEC_STORE);
+        return launch_status();
+    }
+    // A rows past the vectors are never written; they only feed results that
+    // are never stored.
+    hipLaunchKernelGGL(vec_prep_blocks_kernel, dim3((unsigned)(((long)V * KB * 4 + 255) / 256)), dim3(256), 0, stream,
+                       x, xstride, V, KB, A, inv, ssq);
+    GPHQ_TRY(launch_status());
+    if (epi == VEC_ADD) return norm ? launch_vecs<VEC_ADD, true>(fmt, a, stream)
+                                    : launch_vecs<VEC_ADD, false>(fmt, a, stream);
+    if (epi == VEC_SWIGLU) return norm ? launch_vecs<VEC_SWIGLU, true>(fmt, a, stream)
+                                       : launch_vecs<VEC_SWIGLU, false>(fmt, a, stream);
+    return norm ? launch_vecs<VEC_STORE, true>(fmt, a, stream) : launch_vecs<VEC_STORE, false>(fmt, a, stream);
 }
 
 // y[v*ystride + j] for v < V (gphq_gemv_vec). Arguments were validated by the caller.

@@ -105,6 +105,28 @@ def test_formats_lanes_against_float64_and_serial(fmt, lanes, k, n):
         assert rel_s <= 1e-5, (v, rel_s)
 
 
+@pytest.mark.parametrize("fmt", [orc.FMT_Q8, orc.FMT_Q8B, orc.FMT_Q8B_F32, orc.FMT_Q4])
+@pytest.mark.parametrize("k,n", [(32, 1), (64, 17), (96, 15), (544, 16), (2080, 40), (3104, 4097), (4128, 33),
+                                 (8256, 50)])
+def test_slice_and_pass_edges(fmt, k, n):
+    """Partial last slices and lines, block counts that leave scales unaligned,
+    K in one to five passes and a row tile past N, at each arrangement of the
+    vectors (one tile, a hi/lo pair, three and four tiles)."""
+    rng = np.random.default_rng(fmt + k + n)
+    codes, scales = make_weights(fmt, rng, n, k)
+    w = [1, 7, 8, 9, 16, 17, 24, 25, 32] if n < 1000 else [5, 12, 20, 32]
+    x = rng.standard_normal((32, k)).astype(np.float32)
+    x[:, ::37] *= 1e3
+    want = {}
+    for lanes in w:
+        got = run_vec(fmt, codes, scales, x[:lanes].ravel(), lanes, k, n).reshape(lanes, n)
+        for v in {0, lanes // 2, lanes - 1}:
+            if v not in want:
+                want[v] = orc.gemv_f64(fmt, codes, scales, x[v], k, n)[0]
+            _, rel, finite = vector_error(want[v], got[v])
+            assert finite and rel <= 1e-5, (lanes, v, rel)
+
+
 def test_strides_leave_gaps_untouched():
     k, n, lanes, xs, ys = 512, 48, 5, 600, 64
     rng = np.random.default_rng(3)
