@@ -471,379 +471,6 @@ __global__ __launch_bounds__(64 * WM * WN * SK) void i8gemm_kernel(const I8GemmA
     }
 }
 
-// LDS-staged variant for larger M: a block owns a BM x BN output tile; per
-// stage the block copies BKT K-tiles of its A rows and B columns (1 KiB
-// fragments, contiguous in the tile layout) from global memory into LDS with
-// 16-byte loads, double buffered: the next stage's global loads are in flight
-// while the wavefronts multiply the current stage out of LDS. Each fragment
-// then crosses the L2 -> CU path once per block instead of once per wavefront.
-template <int BM, int BN, int WM, int WN, int BKT>
-__global__ __launch_bounds__(64 * WM * WN) void i8gemm_lds_kernel(const I8GemmArgs a) {
-    constexpr int NT_ = 64 * WM * WN;
-    constexpr int TM = BM / 16 / WM, TN = BN / 16 / WN;
-    constexpr int AG = (BM / 16) * BKT, BG = (BN / 16) * BKT;  // 1 KiB groups per stage
-    constexpr int CH = (AG + BG) * 64;                          // 16-byte chunks per stage
-    constexpr int PER = (CH + NT_ - 1) / NT_;
-    __shared__ i32x4 lds[2][AG + BG][64];
-
-    const int G = a.gridM * a.gridN;
-    const int b = blockIdx.x;
-    int logical = b;
-    if (G % 8 == 0) logical = (b % 8) * (G / 8) + b / 8;
-    const int bm = logical % a.gridM, bn = logical / a.gridM;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wm = wv / WN, wn = wv % WN;
-    const int MT = (a.M + 15) >> 4, KT = a.KT;
-    const int rt0 = bm * (BM / 16), ct0 = a.tileN0 + bn * (BN / 16);
-
-    auto fetch = [&](int kt0, i32x4 (&reg)[PER]) {
-#pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            const int c = tid + p * NT_;
-            reg[p] = i32x4{0, 0, 0, 0};
-            if (c < CH) {
-                const int g = c >> 6, l = c & 63;
-                const int kk = (g < AG) ? (g % BKT) : ((g - AG) % BKT);
-                const int kt = kt0 + kk;
-                if (kt < KT) {
-                    if (g < AG) {
-                        const int rt = min(rt0 + g / BKT, MT - 1);
-                        reg[p] = *(const i32x4 *)(a.A + ((size_t)rt * KT + kt) * 1024 + (size_t)l * 16);
-                    } else {
-                        const int ct = min(ct0 + (g - AG) / BKT, a.NT - 1);
-                        reg[p] = __builtin_nontemporal_load(
-                            (const i32x4 *)(a.B + ((size_t)ct * KT + kt) * 1024 + (size_t)l * 16));
-                    }
-                }
-            }
-        }
-    };
-    auto stash = [&](int buf, const i32x4 (&reg)[PER]) {
-#pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            const int c = tid + p * NT_;
-            if (c < CH) lds[buf][c >> 6][c & 63] = reg[p];
-        }
-    };
-
-    i32x4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
-
-    i32x4 reg[PER];
-    fetch(0, reg);
-    stash(0, reg);
-    __syncthreads();
-    int buf = 0;
-    for (int kt0 = 0; kt0 < KT; kt0 += BKT) {
-        const bool more = kt0 + BKT < KT;
-        if (more) fetch(kt0 + BKT, reg);
-#pragma unroll
-        for (int kk = 0; kk < BKT; ++kk) {
-            i32x4 fa[TM], fb[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i] = lds[buf][(wm * TM + i) * BKT + kk][lane];
-#pragma unroll
-            for (int j = 0; j < TN; ++j) fb[j] = lds[buf][AG + (wn * TN + j) * BKT + kk][lane];
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) stash(buf ^ 1, reg);
-        __syncthreads();
-        buf ^= 1;
-    }
-
-    // Scales first, unconditionally, as in i8gemm_kernel's epilogue.
-    float rsc[TM][4], csc[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            rsc[i][e] = a.rowScale[min((rt0 + wm * TM + i) * 16 + 4 * (lane >> 4) + e, a.M - 1)];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int col = (ct0 + wn * TN + j) * 16 + (lane & 15);
-        csc[j] = a.colScale[col >= a.c0 && col < a.c1 ? col : a.c0];
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int col = (ct0 + wn * TN + j) * 16 + (lane & 15);
-        if (col < a.c0 || col >= a.c1) continue;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = (rt0 + wm * TM + i) * 16 + 4 * (lane >> 4) + e;
-                if (row < a.M)
-                    a.dst[(size_t)row * a.stride + col] = __fmul_rn(__fmul_rn((float)acc[i][j][e], csc[j]), rsc[i][e]);
-            }
-        }
-    }
-}
-
-// Skinny-M variant (up to 16 * NWV * RT activation rows per block, one block
-// per NTB weight column tiles; KT a multiple of SB). Every
-// operand fragment goes to LDS with a direct-to-LDS load
-// (global_load_lds_dwordx4: one 1 KiB fragment per wavefront instruction, no
-// registers held while in flight) into a ring of NS stages of SB K-steps; the
-// stage NS - 1 ahead is requested as each stage starts. Each wavefront owns
-// RT row tiles of A and loads their fragments itself; the NTB column tiles of
-// B are shared, each wavefront loading an equal share. Loads return in issue
-// order, so the wait at a stage's start is a count (the loads of the NS - 2
-// stages after it may stay in flight). The barrier is s_barrier with
-// compiler-only fences around it (ring_barrier; a __syncthreads fence would
-// wait for every load in flight), after lgkmcnt(0)
-// so that the previous stage's LDS reads have finished before its slot is
-// refilled.
-template <int NWV, int RT, int NTB, int SB, int NS>
-__global__ __launch_bounds__(64 * NWV) void i8gemm_skinny_kernel(const I8GemmArgs a) {
-    constexpr int FB = NTB * SB;           // B fragments per stage
-    constexpr int FA = NWV * RT * SB;      // A fragments per stage
-    static_assert(FB % NWV == 0, "every wavefront issues the same number of stage loads");
-    constexpr int DB = FB / NWV;           // B loads per wavefront and stage
-    constexpr int D = DB + RT * SB;        // loads per wavefront and stage
-    static_assert(D * (NS - 2) < 64, "in-flight loads beyond the vmcnt range");
-    __shared__ i32x4 ring[NS][FB + FA][64];
-
-    const int G = a.gridM * a.gridN;
-    const int b = blockIdx.x;
-    int logical = b;
-    if (G % 8 == 0) logical = (b % 8) * (G / 8) + b / 8;
-    const int bm = logical % a.gridM, bn = logical / a.gridM;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int MT = (a.M + 15) >> 4, KT = a.KT;
-    const int S = KT / SB;
-    const int mt0 = (bm * NWV + wv) * RT;
-    const int nt0 = a.tileN0 + bn * NTB;
-
-    // Sources of this wavefront's loads at stage 0, in ring order: its B share
-    // (fragment f = wv + NWV * d is column tile f / SB, K-step f % SB), then its
-    // own A fragments (row tile i, K-step kk at FB + (wv * RT + i) * SB + kk).
-    const int8_t *src[D];
-    int dst[D];
-#pragma unroll
-    for (int d = 0; d < DB; ++d) {
-        const int f = wv + NWV * d;
-        src[d] = a.B + ((size_t)min(nt0 + f / SB, a.NT - 1) * KT + f % SB) * 1024 + (size_t)lane * 16;
-        dst[d] = f;
-    }
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int kk = 0; kk < SB; ++kk) {
-            const int d = DB + i * SB + kk;
-            src[d] = a.A + ((size_t)min(mt0 + i, MT - 1) * KT + kk) * 1024 + (size_t)lane * 16;
-            dst[d] = FB + (wv * RT + i) * SB + kk;
-        }
-    auto stage_load = [&](int s) {
-        const int slot = s % NS;
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-            lds_dma16(src[d] + (size_t)s * SB * 1024, &ring[slot][dst[d]][0]);
-    };
-
-    i32x4 acc[RT][NTB];
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int j = 0; j < NTB; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
-
-#pragma unroll
-    for (int p = 0; p < NS - 1; ++p)
-        if (p < S) stage_load(p);
-    for (int s = 0; s < S; ++s) {
-        // Loads of stages s + 1 .. min(S, s + NS - 1) - 1 may remain in flight.
-        const int after = min(S - 1 - s, NS - 2);
-        if (after == NS - 2)
-            wait_vm_lgkm0<D * (NS - 2)>();
-        else if (after == 1)
-            wait_vm_lgkm0<D>();
-        else
-            wait_vm_lgkm0<0>();
-        ring_barrier();
-        if (s + NS - 1 < S) stage_load(s + NS - 1);
-        const int slot = s % NS;
-#pragma unroll
-        for (int kk = 0; kk < SB; ++kk) {
-            i32x4 fa[RT], fb[NTB];
-#pragma unroll
-            for (int i = 0; i < RT; ++i) fa[i] = ring[slot][FB + (wv * RT + i) * SB + kk][lane];
-#pragma unroll
-            for (int j = 0; j < NTB; ++j) fb[j] = ring[slot][j * SB + kk][lane];
-#pragma unroll
-            for (int i = 0; i < RT; ++i)
-#pragma unroll
-                for (int j = 0; j < NTB; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-    }
-
-    // Epilogue as in i8gemm_kernel: scales first, then the stores.
-    float rsc[RT][4], csc[NTB];
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) rsc[i][e] = a.rowScale[min((mt0 + i) * 16 + 4 * (lane >> 4) + e, a.M - 1)];
-#pragma unroll
-    for (int j = 0; j < NTB; ++j) {
-        const int col = (nt0 + j) * 16 + (lane & 15);
-        csc[j] = a.colScale[col >= a.c0 && col < a.c1 ? col : a.c0];
-    }
-#pragma unroll
-    for (int j = 0; j < NTB; ++j) {
-        const int col = (nt0 + j) * 16 + (lane & 15);
-        if (col < a.c0 || col >= a.c1) continue;
-#pragma unroll
-        for (int i = 0; i < RT; ++i) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = (mt0 + i) * 16 + 4 * (lane >> 4) + e;
-                if (row < a.M)
-                    a.dst[(size_t)row * a.stride + col] = __fmul_rn(__fmul_rn((float)acc[i][j][e], csc[j]), rsc[i][e]);
-            }
-        }
-    }
-}
-
-// Large-M variant: BM x BN block tiles (WGM x WGN wavefronts, each a grid of
-// 32 x 32 v_mfma_i32_32x32x32_i8 tiles), 128-deep K steps staged through LDS
-// as 128-byte rows with the row-swizzled 16-byte chunks of the FP16 big-tile
-// GEMM, double-buffered with the next step's global loads in flight;
-// XCD-grouped tile order. Exact int32 sums, so the bits equal the other
-// kernels'. Operands come in the tile layout (two 64-deep groups per step).
-// Epilogue: (float32(sum) * colScale) * rowScale, stored.
-template <int BM, int BN, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_big_kernel(const I8GemmArgs a) {
-    typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
-    constexpr int NT = 64 * WGM * WGN;
-    constexpr int TI = BM / WGM / 32, TJ = BN / WGN / 32;
-    constexpr int AL = BM * 8 / NT, BL = BN * 8 / NT;  // 16-byte units per thread and step
-    static_assert(AL >= 1 && BL >= 1, "loader split");
-    __shared__ i32x4 As[2][BM * 8];
-    __shared__ i32x4 Bs[2][BN * 8];
-    int bm, bn;
-    tile_order(blockIdx.x, a.gridM, a.gridN, bm, bn);
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int wm = wv / WGN, wn = wv % WGN;
-    const int rt0 = bm * (BM / 16), ct0 = a.tileN0 + bn * (BN / 16);
-    const int MT = (a.M + 15) >> 4, KT = a.KT;
-    const int steps = (KT + 1) / 2;
-    // Unit u = i*NT + t of a step is 16-row tile u/128, group (u/64)%2 of the
-    // step, lane slot u%64 (row slot%16, K bytes 16*(slot/16) of the group).
-    auto gload = [&](const int8_t *base, int tile0, int tiles, int u, int st) {
-        i32x4 v = i32x4{0, 0, 0, 0};
-        const int kt = 2 * st + ((u >> 6) & 1);
-        if (kt < KT)
-            v = *(const i32x4 *)(base + ((size_t)min(tile0 + (u >> 7), tiles - 1) * KT + kt) * 1024 +
-                                 (size_t)(u & 63) * 16);
-        return v;
-    };
-    auto lidx = [](int u) {
-        const int r = (u >> 7) * 16 + (u & 15);
-        return r * 8 + big_swz(r, ((u >> 6) & 1) * 4 + ((u & 63) >> 4));
-    };
-    const int aRows = MT, bRows = a.NT;
-    i32x4 ar[AL], br[BL];
-    auto load = [&](int st) {
-#pragma unroll
-        for (int i = 0; i < AL; ++i) ar[i] = gload(a.A, rt0, aRows, i * NT + t, st);
-#pragma unroll
-        for (int i = 0; i < BL; ++i) br[i] = gload(a.B, ct0, bRows, i * NT + t, st);
-    };
-    auto store = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < AL; ++i) As[buf][lidx(i * NT + t)] = ar[i];
-#pragma unroll
-        for (int i = 0; i < BL; ++i) Bs[buf][lidx(i * NT + t)] = br[i];
-    };
-    i32x16 acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = i32x16{};
-    load(0);
-    store(0);
-    if (steps > 1) load(1);
-    __syncthreads();
-    const int fr = lane & 31, fh = lane >> 5;
-    // With two wavefronts per SIMD (8 per block), the second wavefront of each
-    // SIMD stores the next step's tiles before its MFMAs and the first after
-    // them, so the SIMD's MFMA pipe is fed by one while the other stores
-    // (measured: M = 512, 54 -> 52 us).
-    const bool early = NT >= 512 && wv >= NT / 128;
-    for (int st = 0; st < steps; ++st) {
-        const int cur = st & 1;
-        if (early && st + 1 < steps) {
-            store(cur ^ 1);
-            if (st + 2 < steps) load(st + 2);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int c = 2 * s + fh;
-            i32x4 fa[TI], fb[TJ];
-#pragma unroll
-            for (int i = 0; i < TI; ++i) {
-                const int r = wm * (32 * TI) + 32 * i + fr;
-                fa[i] = As[cur][r * 8 + big_swz(r, c)];
-            }
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-                const int r = wn * (32 * TJ) + 32 * j + fr;
-                fb[j] = Bs[cur][r * 8 + big_swz(r, c)];
-            }
-#pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int j = 0; j < TJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        if (!early && st + 1 < steps) {
-            store(cur ^ 1);
-            if (st + 2 < steps) load(st + 2);
-        }
-        __syncthreads();
-    }
-    // Epilogue as MulPanelsI8: (float32(sum) * colScale) * rowScale. Every
-    // scale of the lane's outputs is read up front, unconditionally (rows past
-    // M read the last row; they are not written): read inside the store loop,
-    // or under a branch, each scale costs a wait, and the wait also drains
-    // every store issued before it (stores may alias the scales as far as the
-    // compiler knows, and the counter it waits on counts stores too).
-    float rsc[TI][16];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-            rsc[i][e] = a.rowScale[min((rt0 + (wm * TI + i) * 2) * 16 + 8 * (e >> 2) + 4 * fh + (e & 3), a.M - 1)];
-    // The column scales too (a column outside [c0, c1) reads c0's and is not
-    // written): a load after a store waits for the store as well.
-    float csc[TJ];
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-        const int col = (ct0 + (wn * TJ + j) * 2) * 16 + fr;
-        csc[j] = a.colScale[col >= a.c0 && col < a.c1 ? col : a.c0];
-    }
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-        const int col = (ct0 + (wn * TJ + j) * 2) * 16 + fr;
-        if (col < a.c0 || col >= a.c1) continue;
-        const float cs = csc[j];
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = (rt0 + (wm * TI + i) * 2) * 16 + 8 * (e >> 2) + 4 * fh + (e & 3);
-                if (row < a.M)
-                    a.dst[(size_t)row * a.stride + col] = __fmul_rn(__fmul_rn((float)acc[i][j][e], cs), rsc[i][e]);
-            }
-    }
-}
-
 // Epilogue of the direct-to-LDS kernels, as in i8gemm_kernel: lane l of a
 // 16 x 16 tile holds rows 4 (l / 16) + e, column l % 16; scales first, then
 // the stores. mt0 / nt0: the wavefront's first row and column tile.
@@ -947,113 +574,24 @@ __device__ __forceinline__ void dma_epilogue(const I8GemmArgs &a, const i32x4 (&
         dma_epilogue_stores<TI, TJ, EPI, 0>(a, acc, mt0, nt0, lane, rsc, csc);
 }
 
-// Direct-to-LDS variant: BM x BN block tiles (WGM x WGN wavefronts, each a
-// grid of 16 x 16 v_mfma_i32_16x16x64_i8 tiles), a ring of NS stages of one
-// 64-deep K-step, every operand fragment (the tile layout's 1 KiB group of
-// 16 rows x 64 bytes) loaded with global_load_lds_dwordx4 and read back by
-// the lanes that own it (lane l at byte 16 l: no bank conflicts). BROWS (the
+// The direct-to-LDS kernels below: BM x BN block tiles, WGM x WGN wavefronts
+// each with a grid of 16 x 16 v_mfma_i32_16x16x64_i8 tiles, a ring of NS LDS
+// stages. Every operand fragment (the tile layout's 1 KiB group of 16 rows x
+// 64 bytes) loads with one global_load_lds_dwordx4 and is read back by the
+// lanes that own it (lane l at byte 16 l: no bank conflicts). BROWS (the
 // batched pass) takes A as row tiles (rowtile_offset) and B from row-major
 // rows (a.K bytes each, K a multiple of 64): each fragment is gathered into
 // the same LDS image, lane l reading row l % 16 at byte 16 (l / 16) of the
-// step (for A inside one 1 KiB group). The stage NS - 1 ahead is
-// requested as each stage starts; the wait is a count, as in the skinny
-// kernel. When the fragments of a stage do not split evenly over the
-// wavefronts, the first F % NW issue one more. Epilogue (float32(sum) *
-// colScale) * rowScale, then a store, an fp32 atomic add into dst
-// (I8_EPI_ADD: one owner per element, so exactly dst + v) or the SwiGLU of
-// interleaved gate/up columns into dst[row][col / 2] (I8_EPI_SWIGLU, the
-// neighbouring column's value by DPP).
-template <int BM, int BN, int WGM, int WGN, int NS, bool BROWS, int EPI>
-__global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_dma_kernel(const I8GemmArgs a) {
-    constexpr int NW = WGM * WGN;
-    constexpr int FA = BM / 16, FB = BN / 16, F = FA + FB;  // fragments per stage
-    constexpr int DMAX = (F + NW - 1) / NW, DREM = F % NW;  // loads per wavefront and stage
-    constexpr int TI = BM / 16 / WGM, TJ = BN / 16 / WGN;
-    static_assert(TI * 16 * WGM == BM && TJ * 16 * WGN == BN, "wave grid");
-    static_assert(DMAX * (NS - 2) < 64, "in-flight loads beyond the vmcnt range");
-    __shared__ i32x4 ring[NS][F][64];
-    int bm, bn;
-    tile_order(blockIdx.x, a.gridM, a.gridN, bm, bn);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wm = wv / WGN, wn = wv % WGN;
-    const int rt0 = bm * FA, ct0 = a.tileN0 + bn * FB;
-    const int MT = (a.M + 15) >> 4, KT = a.KT;
-    // Loads of this wavefront: fragment f = wv + NW * d (A tiles first, then B).
-    const bool full = DREM == 0 || wv < DREM;  // issues DMAX loads per stage, else DMAX - 1
-    const int8_t *src[DMAX];
-    int dst[DMAX];
-#pragma unroll
-    for (int d = 0; d < DMAX; ++d) {
-        const int f = min(wv + NW * d, F - 1);
-        dst[d] = f;
-        if (f < FA) {
-            // With BROWS, A comes as row tiles (rowtile_offset): lane l gathers
-            // row l % 16's bytes 16 (l / 16) of the group.
-            src[d] = a.A + (size_t)min(rt0 + f, MT - 1) * KT * 1024 +
-                     (BROWS ? (size_t)(lane & 15) * 64 + (lane >> 4) * 16 : (size_t)lane * 16);
-        } else if constexpr (BROWS) {
-            src[d] = a.B + (size_t)min((ct0 + (f - FA)) * 16 + (lane & 15), a.N - 1) * a.K + (lane >> 4) * 16;
-        } else {
-            src[d] = a.B + (size_t)min(ct0 + (f - FA), a.NT - 1) * KT * 1024 + (size_t)lane * 16;
-        }
-    }
-    auto stage_load = [&](int s) {
-        const int slot = s % NS;
-#pragma unroll
-        for (int d = 0; d < DMAX; ++d)
-            if (d < DMAX - 1 || full)
-                lds_dma16(src[d] + (size_t)s * (BROWS && dst[d] >= FA ? 64 : 1024), &ring[slot][dst[d]][0]);
-    };
-    i32x4 acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int p = 0; p < NS - 1; ++p)
-        if (p < KT) stage_load(p);
-    for (int s = 0; s < KT; ++s) {
-        // Loads of the stages after s already requested may stay in flight.
-        const int after = min(KT - 1 - s, NS - 2);
-        if (after == NS - 2) {
-            if (full)
-                wait_vm_lgkm0<DMAX * (NS - 2)>();
-            else
-                wait_vm_lgkm0<(DMAX - 1) * (NS - 2)>();
-        } else if (after == 1) {
-            if (full)
-                wait_vm_lgkm0<DMAX>();
-            else
-                wait_vm_lgkm0<DMAX - 1>();
-        } else {
-            wait_vm_lgkm0<0>();
-        }
-        ring_barrier();
-        if (s + NS - 1 < KT) stage_load(s + NS - 1);
-        const int slot = s % NS;
-        i32x4 fa[TI], fb[TJ];
-#pragma unroll
-        for (int i = 0; i < TI; ++i) fa[i] = ring[slot][wm * TI + i][lane];
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) fb[j] = ring[slot][FA + wn * TJ + j][lane];
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
-    }
-    dma_epilogue<TI, TJ, EPI>(a, acc, rt0 + wm * TI, ct0 + wn * TJ, lane);
-}
-
-template <int BM, int BN, int WGM, int WGN, int NS, bool BROWS = false, int EPI = I8_EPI_STORE>
-static int launch_i8gemm_dma(I8GemmArgs a, hipStream_t stream) {
-    const int tiles = (a.c1 + 15) / 16 - a.tileN0;
-    a.gridN = (tiles * 16 + BN - 1) / BN;
-    a.gridM = (a.M + BM - 1) / BM;
-    hipLaunchKernelGGL((i8gemm_dma_kernel<BM, BN, WGM, WGN, NS, BROWS, EPI>), dim3((unsigned)(a.gridM * a.gridN)),
-                       dim3(64 * WGM * WGN), 0, stream, a);
-    return launch_status();
-}
+// step (for A inside one 1 KiB group). Loads return in issue order, so a wait
+// is a count of the loads issued after the stage it waits for; the barrier is
+// s_barrier with compiler-only fences around it (ring_barrier; a
+// __syncthreads fence would wait for every load in flight). When the
+// fragments of a stage do not split evenly over the wavefronts that load
+// them, the first ones issue one more. Epilogue (float32(sum) * colScale) *
+// rowScale, then a store, an fp32 atomic add into dst (I8_EPI_ADD: one owner
+// per element, so exactly dst + v) or the SwiGLU of interleaved gate/up
+// columns into dst[row][col / 2] (I8_EPI_SWIGLU, the neighbouring column's
+// value by DPP).
 
 // vmcnt(PER * min(after, MAXA)) and lgkmcnt(0).
 template <int PER, int MAXA>
@@ -1068,24 +606,23 @@ __device__ __forceinline__ void wait_stages_n(int after) {
     }
 }
 
-// Ping-pong variant of i8gemm_dma_kernel (8 wavefronts, two per SIMD: a
-// probe of the hardware wave id on MI355X places wavefronts w and w + 4 of a
-// 512-thread block on one SIMD). The wavefronts of group 0 (0-3) and group 1
-// (4-7) run half a K step apart: while one group issues its MFMAs for a step
-// (at raised wave priority), the other requests the ring stage NS - 1 ahead,
-// reads its fragments of the step from LDS and waits for its share of the
-// next stage; a barrier ends each half. Group 1 starts one barrier late and
+// Ping-pong schedule, one 64-deep K-step per stage (8 wavefronts, two per
+// SIMD: a probe of the hardware wave id on MI355X places wavefronts w and w + 4
+// of a 512-thread block on one SIMD). The wavefronts of group 0 (0-3) and
+// group 1 (4-7) run half a K step apart: while one group issues its MFMAs for a
+// step (at raised wave priority), the other requests the ring stage NS - 1
+// ahead, reads its fragments of the step from LDS and waits for its share of
+// the next stage; a barrier ends each half. Group 1 starts one barrier late and
 // group 0 ends with one extra, so every wavefront passes the same number of
 // barriers (2 KT + 2). Ordering: a wavefront's share of stage s + 1 is
 // complete, and its reads of stage s returned, before the barrier that ends
 // its memory half of step s; so both groups' shares of a stage are in LDS
 // before the barrier after which group 0 reads it, and the slot that stage
 // s + NS - 1 overwrites (stage s - 1's) was last read before the barrier
-// preceding the memory half that requests it. Measured on MI355X against
-// i8gemm_dma_kernel: the 4096-row int8 pass 54.2-54.4 -> 53.4-53.7 ms (256 x
-// 256 tiles, NS = 5), config 2 at M = 512 43.6-44.0 -> 40.8-42.9 us (128 x
-// 192 tiles, NS = 6); NS = 4 for the pass gave no gain.
-template <int BM, int BN, int WGM, int WGN, int NS, bool BROWS, int EPI>
+// preceding the memory half that requests it. 256 x 256 tiles of the tile
+// layout, NS = 5, K = 4096, N = 12288, M = 4096: 160 us (2.58 POPS; 387 us with
+// both operands staged through registers).
+template <int BM, int BN, int WGM, int WGN, int NS>
 __global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_pp_kernel(const I8GemmArgs a) {
     constexpr int NW = WGM * WGN;
     static_assert(NW == 8, "two groups of four wavefronts");
@@ -1110,10 +647,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_pp_kernel(const I8GemmA
         const int f = min(wv + NW * d, F - 1);
         dst[d] = f;
         if (f < FA) {
-            src[d] = a.A + (size_t)min(rt0 + f, MT - 1) * KT * 1024 +
-                     (BROWS ? (size_t)(lane & 15) * 64 + (lane >> 4) * 16 : (size_t)lane * 16);
-        } else if constexpr (BROWS) {
-            src[d] = a.B + (size_t)min((ct0 + (f - FA)) * 16 + (lane & 15), a.N - 1) * a.K + (lane >> 4) * 16;
+            src[d] = a.A + (size_t)min(rt0 + f, MT - 1) * KT * 1024 + (size_t)lane * 16;
         } else {
             src[d] = a.B + (size_t)min(ct0 + (f - FA), a.NT - 1) * KT * 1024 + (size_t)lane * 16;
         }
@@ -1123,7 +657,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_pp_kernel(const I8GemmA
 #pragma unroll
         for (int d = 0; d < DMAX; ++d)
             if (d < DMAX - 1 || full)
-                lds_dma16(src[d] + (size_t)s * (BROWS && dst[d] >= FA ? 64 : 1024), &ring[slot][dst[d]][0]);
+                lds_dma16(src[d] + (size_t)s * 1024, &ring[slot][dst[d]][0]);
     };
     auto wait_stages = [&](int after) {
         if (full)
@@ -1172,46 +706,263 @@ __global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_pp_kernel(const I8GemmA
         barrier();
     }
     if (grp == 0) barrier();
+    dma_epilogue<TI, TJ, I8_EPI_STORE>(a, acc, rt0 + wm * TI, ct0 + wn * TJ, lane);
+}
+
+// The ping-pong schedule for row-major weights (the batched pass): a 64-deep
+// step takes half a 128-byte line of each weight row, and loads of half lines
+// (16 rows x 64 bytes an instruction) held the schedule to 1.67 POPS (Qwen3-8B
+// gate/up at 4096 rows, SwiGLU; the tile layout's whole groups run 2.58). Whole
+// lines: 498 -> 465 us with the activation pack, 1.85 POPS. B comes in pieces
+// of two K-steps: 8 rows x 128 bytes an instruction, lane l taking chunk (l % 8)
+// ^ ((row / 2) % 8) of row l / 8, so that a fragment's 16 rows at one chunk sit on distinct
+// banks. LDS holds four A stages and three B pieces; a step requests A's stage
+// three ahead and, when even, B's piece two ahead (the slot of the piece
+// before this one, whose last reads precede the barrier before the request, as
+// in i8gemm_pp_kernel). At the end of a memory half the wavefront's loads older
+// than A's stage s + 1 are complete, so may remain in flight: for an even step
+// B's piece of step s - 2, A's of s - 1, and both of s; for an odd one A's and
+// B's of s - 1 and A's of s. The last steps, whose requests run out, wait for
+// all. A piece past K (an odd step count) reads its row's first half twice.
+template <int BN, int EPI>
+__global__ __launch_bounds__(512) void i8gemm_rows_kernel(const I8GemmArgs a) {
+    constexpr int BM = 256, WGM = 4, WGN = 2;
+    constexpr int TI = BM / 16 / WGM, TJ = BN / 16 / WGN;
+    constexpr int LA = BM / 16 / 8, LB = BN / 8 / 8;  // loads per wavefront: A per step, B per piece
+    constexpr int NA = 4, NB = 3;
+    // One array: with two the compiler waits for every direct-to-LDS load into
+    // either before it reads from one.
+    __shared__ i32x4 lds[NA * BM * 4 + NB * BN * 8];
+    i32x4 *const As = lds, *const Bs = lds + NA * BM * 4;  // [NA][BM / 16][64]; [NB][row][8 chunks, swizzled]
+    int bm, bn;
+    tile_order(blockIdx.x, a.gridM, a.gridN, bm, bn);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wv >> 2;
+    const int wm = wv / WGN, wn = wv % WGN;
+    const int rt0 = bm * (BM / 16), ct0 = a.tileN0 + bn * (BN / 16);
+    const int MT = (a.M + 15) >> 4, KT = a.KT;
+    const int pieces = (KT + 1) / 2;
+    const int8_t *asrc[LA], *bsrc[LB];
+    const int brow = lane >> 3;
+    int bchunk[LB];
+#pragma unroll
+    for (int d = 0; d < LA; ++d)
+        asrc[d] = a.A + (size_t)min(rt0 + wv + 8 * d, MT - 1) * KT * 1024 + (size_t)(lane & 15) * 64 + (lane >> 4) * 16;
+#pragma unroll
+    for (int d = 0; d < LB; ++d) {
+        const int r = 8 * (wv + 8 * d) + brow;  // row of the block's tile
+        bchunk[d] = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+        bsrc[d] = a.B + (size_t)min(ct0 * 16 + r, a.N - 1) * a.K;
+    }
+    auto aload = [&](int s) {
+#pragma unroll
+        for (int d = 0; d < LA; ++d) lds_dma16(asrc[d] + (size_t)s * 1024, &As[(s % NA) * (BM * 4) + 64 * (wv + 8 * d)]);
+    };
+    auto bload = [&](int p) {
+        const bool half = 2 * p + 1 >= KT;
+#pragma unroll
+        for (int d = 0; d < LB; ++d)
+            lds_dma16(bsrc[d] + (size_t)p * 128 + (half ? bchunk[d] & 63 : bchunk[d]), &Bs[(p % NB) * (BN * 8) + 64 * (wv + 8 * d)]);
+    };
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        ring_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    i32x4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+    bload(0);
+    aload(0);
+    if (pieces > 1) bload(1);
+    if (KT > 1) aload(1);
+    if (KT > 2) aload(2);
+    wait_vm_lgkm0<0>();
+    barrier();
+    if (grp == 1) barrier();
+    const int fr = lane & 15, fg = lane >> 4;
+    i32x4 fa[TI], fb[TJ];
+    auto step = [&](int s, int odd) {
+        // Memory half.
+        if (s + 3 < KT) aload(s + 3);
+        if (!odd && s / 2 + 2 < pieces) bload(s / 2 + 2);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) fa[i] = As[(s % NA) * (BM * 4) + 64 * (wm * TI + i) + lane];
+        const int slot = (s / 2) % NB;
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int r = (wn * TJ + j) * 16 + fr;
+            fb[j] = Bs[slot * (BN * 8) + r * 8 + ((4 * odd + fg) ^ ((r >> 1) & 7))];
+        }
+        if (s + 4 < KT) {
+            if (odd) wait_vm_lgkm0<2 * LA + LB>();
+            else wait_vm_lgkm0<2 * LA + 2 * LB>();
+        } else {
+            wait_vm_lgkm0<0>();
+        }
+        barrier();
+        // MFMA half.
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        barrier();
+    };
+    for (int s = 0; s < KT; s += 2) {
+        step(s, 0);
+        if (s + 1 < KT) step(s + 1, 1);
+    }
+    if (grp == 0) barrier();
     dma_epilogue<TI, TJ, EPI>(a, acc, rt0 + wm * TI, ct0 + wn * TJ, lane);
 }
 
-template <int BM, int BN, int WGM, int WGN, int NS, bool BROWS = false, int EPI = I8_EPI_STORE>
+template <int BN, int EPI>
+static int launch_i8gemm_rows(I8GemmArgs a, hipStream_t stream) {
+    const int tiles = (a.c1 + 15) / 16 - a.tileN0;
+    a.gridN = (tiles * 16 + BN - 1) / BN;
+    a.gridM = (a.M + 255) / 256;
+    hipLaunchKernelGGL((i8gemm_rows_kernel<BN, EPI>), dim3((unsigned)(a.gridM * a.gridN)), dim3(512), 0, stream, a);
+    return launch_status();
+}
+
+template <int BM, int BN, int WGM, int WGN, int NS>
 static int launch_i8gemm_pp(I8GemmArgs a, hipStream_t stream) {
     const int tiles = (a.c1 + 15) / 16 - a.tileN0;
     a.gridN = (tiles * 16 + BN - 1) / BN;
     a.gridM = (a.M + BM - 1) / BM;
-    hipLaunchKernelGGL((i8gemm_pp_kernel<BM, BN, WGM, WGN, NS, BROWS, EPI>), dim3((unsigned)(a.gridM * a.gridN)),
+    hipLaunchKernelGGL((i8gemm_pp_kernel<BM, BN, WGM, WGN, NS>), dim3((unsigned)(a.gridM * a.gridN)),
                        dim3(64 * WGM * WGN), 0, stream, a);
     return launch_status();
 }
 
-template <int BM, int BN, int WGM, int WGN>
-static int launch_i8gemm_big(I8GemmArgs a, hipStream_t stream) {
+// BM x BN block tiles with the roles split: NP wavefronts only issue
+// direct-to-LDS loads (a ring of NS stages of SB 64-deep K-steps), WGM x WGN
+// wavefronts only multiply. A CU takes 60 bytes a clock from L2 (measured: 125-
+// 143 GB/s, by direct-to-LDS or register loads, from 64 KB in flight), but a
+// wavefront that both issues a stage's loads (16 clocks each on the address
+// path) and multiplies it does one after the other, and kernels built so moved
+// 16 bytes a clock at any M and N (M = 100, K = 4096: 18 us for N = 600 and for
+// N = 3396; 9.9 and 12.1 here). Here the
+// issue, the fragment reads (one K-step ahead, in a second register set) and
+// the MFMAs run beside each other. Every wavefront passes one barrier before
+// the loop and one per stage. Ordering: at the barrier that ends stage s,
+// stage s + 2 is complete (the loaders' wait) and every read of stage s has
+// returned (lgkmcnt(0)); during stage s the multipliers read stage s and the
+// first step of s + 1, and the loaders refill the slot of stage s - 1. K-steps
+// past KT in the last stage load the last step again and are not multiplied.
+template <int BM, int BN, int WGM, int WGN, int NP, int SB, int NS, bool BROWS, int EPI>
+__global__ __launch_bounds__(64 * (WGM * WGN + NP)) void i8gemm_roles_kernel(const I8GemmArgs a) {
+    constexpr int NC = WGM * WGN;
+    constexpr int FA = BM / 16, FB = BN / 16, F = FA + FB;  // fragments per K-step
+    constexpr int FS = F * SB;                              // per stage
+    constexpr int DMAX = (FS + NP - 1) / NP, DREM = FS % NP;
+    constexpr int TI = BM / 16 / WGM, TJ = BN / 16 / WGN;
+    static_assert(TI * 16 * WGM == BM && TJ * 16 * WGN == BN, "wave grid");
+    static_assert(NS >= 4 && DMAX * (NS - 3) < 64, "ring depth");
+    __shared__ i32x4 ring[NS][FS][64];
+    int bm, bn;
+    tile_order(blockIdx.x, a.gridM, a.gridN, bm, bn);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rt0 = bm * FA, ct0 = a.tileN0 + bn * FB;
+    const int MT = (a.M + 15) >> 4, KT = a.KT;
+    const int S = (KT + SB - 1) / SB;
+    if (wv >= NC) {
+        const int pw = wv - NC;
+        const bool full = DREM == 0 || pw < DREM;
+        const int8_t *src[DMAX];
+        int dst[DMAX];
+#pragma unroll
+        for (int d = 0; d < DMAX; ++d) {
+            dst[d] = min(pw + NP * d, FS - 1);
+            const int f = dst[d] % F;
+            if (f < FA) {
+                src[d] = a.A + (size_t)min(rt0 + f, MT - 1) * KT * 1024 +
+                         (BROWS ? (size_t)(lane & 15) * 64 + (lane >> 4) * 16 : (size_t)lane * 16);
+            } else if constexpr (BROWS) {
+                src[d] = a.B + (size_t)min((ct0 + (f - FA)) * 16 + (lane & 15), a.N - 1) * a.K + (lane >> 4) * 16;
+            } else {
+                src[d] = a.B + (size_t)min(ct0 + (f - FA), a.NT - 1) * KT * 1024 + (size_t)lane * 16;
+            }
+        }
+        int slot = 0;
+        auto stage_load = [&](int s) {
+#pragma unroll
+            for (int d = 0; d < DMAX; ++d)
+                if (d < DMAX - 1 || full) {
+                    const int st = min(s * SB + dst[d] / F, KT - 1);
+                    lds_dma16(src[d] + (size_t)st * (BROWS && dst[d] % F >= FA ? 64 : 1024), &ring[slot][dst[d]][0]);
+                }
+            slot = slot + 1 == NS ? 0 : slot + 1;
+        };
+        auto wait_stages = [&](int after) {
+            if (full)
+                wait_stages_n<DMAX, NS - 3>(after);
+            else
+                wait_stages_n<DMAX - 1, NS - 3>(after);
+        };
+        for (int p = 0; p < NS - 1; ++p)
+            if (p < S) stage_load(p);
+        wait_stages(min(S - 2, NS - 3));  // stages 0 and 1
+        ring_barrier();
+        for (int s = 0; s < S; ++s) {
+            if (s + NS - 1 < S) stage_load(s + NS - 1);
+            wait_stages(min(S - 3 - s, NS - 3));
+            ring_barrier();
+        }
+        return;
+    }
+    const int wm = wv / WGN, wn = wv % WGN;
+    i32x4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+    i32x4 fa[2][TI], fb[2][TJ];
+    int rslot = 0, rstep = 0;  // where the next K-step's fragments are
+    auto frags = [&](int set) {
+        const i32x4(*r)[64] = &ring[rslot][rstep * F];
+#pragma unroll
+        for (int i = 0; i < TI; ++i) fa[set][i] = r[wm * TI + i][lane];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) fb[set][j] = r[FA + wn * TJ + j][lane];
+        if (++rstep == SB) {
+            rstep = 0;
+            rslot = rslot + 1 == NS ? 0 : rslot + 1;
+        }
+    };
+    ring_barrier();
+    frags(0);
+    auto step = [&](int k, int set) {
+        if (k + 1 < KT) frags(set ^ 1);
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[set][i], fb[set][j], acc[i][j], 0, 0, 0);
+        if ((k + 1) % SB == 0 || k + 1 == KT) {
+            wait_vm_lgkm0<63>();
+            ring_barrier();
+        }
+    };
+    for (int k = 0; k < KT; k += 2) {
+        step(k, 0);
+        if (k + 1 < KT) step(k + 1, 1);
+    }
+    dma_epilogue<TI, TJ, EPI>(a, acc, rt0 + wm * TI, ct0 + wn * TJ, lane);
+}
+
+template <int BM, int BN, int WGM, int WGN, int NP, int SB, int NS, bool BROWS = false, int EPI = I8_EPI_STORE>
+static int launch_i8gemm_roles(I8GemmArgs a, hipStream_t stream) {
     const int tiles = (a.c1 + 15) / 16 - a.tileN0;
     a.gridN = (tiles * 16 + BN - 1) / BN;
     a.gridM = (a.M + BM - 1) / BM;
-    hipLaunchKernelGGL((i8gemm_big_kernel<BM, BN, WGM, WGN>), dim3((unsigned)(a.gridM * a.gridN)),
-                       dim3(64 * WGM * WGN), 0, stream, a);
-    return launch_status();
-}
-
-template <int BM, int BN, int WM, int WN, int BKT>
-static int launch_i8gemm_lds(I8GemmArgs a, hipStream_t stream) {
-    const int tiles = (a.c1 + 15) / 16 - a.tileN0;
-    a.gridN = (tiles * 16 + BN - 1) / BN;
-    a.gridM = (a.M + BM - 1) / BM;
-    const unsigned blocks = (unsigned)(a.gridM * a.gridN);
-    hipLaunchKernelGGL((i8gemm_lds_kernel<BM, BN, WM, WN, BKT>), dim3(blocks), dim3(64 * WM * WN), 0, stream, a);
-    return launch_status();
-}
-
-template <int NWV, int RT, int NTB, int SB, int NS>
-static int launch_i8gemm_skinny(I8GemmArgs a, hipStream_t stream) {
-    const int tiles = (a.c1 + 15) / 16 - a.tileN0;
-    a.gridN = (tiles + NTB - 1) / NTB;
-    a.gridM = (a.M + 16 * NWV * RT - 1) / (16 * NWV * RT);
-    const unsigned blocks = (unsigned)(a.gridM * a.gridN);
-    hipLaunchKernelGGL((i8gemm_skinny_kernel<NWV, RT, NTB, SB, NS>), dim3(blocks), dim3(64 * NWV), 0, stream, a);
+    hipLaunchKernelGGL((i8gemm_roles_kernel<BM, BN, WGM, WGN, NP, SB, NS, BROWS, EPI>),
+                       dim3((unsigned)(a.gridM * a.gridN)), dim3(64 * (WGM * WGN + NP)), 0, stream, a);
     return launch_status();
 }
 
@@ -1244,25 +995,48 @@ int i8gemm_launch(const int8_t *A, const int8_t *B, const float *rowScale, const
     a.c0 = c0;
     a.c1 = c1;
     a.tileN0 = c0 / 16;
-    // Shapes picked by measurement on MI355X at K = 4096, N = 12288 (M = 512:
-    // 78.5 us with 128 x 64 LDS tiles, 49.0 with 256 x 128 big tiles, 46.1
-    // with 128 x 192, one tile per CU; M = 32 / 64 / 128 / 256: 16.3 / 26 /
-    // 27.6 / 38.5 us before the skinny kernel, 11.6 / 12.5 / 18.5 / 32.5 with
-    // it).
-    // M = 192 / 256 / 384 / 512: 40.6 / 39.4 / 39.7 / 41.1 us with the
-    // register-staged big tiles, 24.0 / 24.5 / 35.5 / 36.4 with the
-    // direct-to-LDS ones.
+    // Up to 16 rows the weights alone bound the product: 32 columns a block, K
+    // split over its wavefronts (M = 8, N = 12288, K = 4096: 10.7 us; 16.8 in
+    // 16 x 16 tiles below).
     if (M <= 16) return launch_i8gemm<1, 2, 1, 2, 4, 4>(a, stream);
-    if (KT % 4 == 0) {  // skinny kernel: whole 4-step stages
-        if (M <= 32) return launch_i8gemm_skinny<2, 1, 3, 4, 4>(a, stream);
-        if (M <= 64) return launch_i8gemm_skinny<4, 1, 3, 4, 3>(a, stream);
-        if (M <= 128) return launch_i8gemm_skinny<4, 2, 3, 4, 3>(a, stream);
+    // Above, one tile per CU at a time, and a tile's time follows its K steps
+    // whatever the rest of the chip does: the tile with the least rounds of
+    // the chip x (steps x time per step + fill and stores) is the fastest.
+    // Nanoseconds per 64-deep step measured on MI355X (KT 12 against 64).
+    // K = 4096, N = 12288, M = 24 / 50 / 100 / 200 / 500 / 1000 / 4096: 13.5 /
+    // 14.2 / 19.6 / 23.8 / 35.9 / 75.3 / 387 us before (tiles chosen by M
+    // alone, each wavefront loading what it multiplies), 12.5 / 13.0 / 15.9 /
+    // 20.0 / 30.8 / 47.7 / 160 with this; N = 3396: 12.2 / 12.9 / 18.1 / 21.8 /
+    // 31.4 / 41.0 / 122 before, 9.3 / 9.4 / 12.1 / 12.8 / 16.2 / 22.1 / 55.6.
+    struct Tile {
+        int bm, bn, ns;
+    };
+    static constexpr Tile tiles[] = {{64, 16, 87},   {64, 32, 92},   {32, 48, 95},   {64, 48, 108},
+                                     {128, 32, 112}, {64, 64, 123},  {128, 48, 133}, {128, 64, 163},
+                                     {128, 96, 177}, {128, 128, 190}, {128, 192, 325}, {256, 256, 560}};
+    int best = 0;
+    long cost = 0;
+    for (int i = 0; i < (int)(sizeof(tiles) / sizeof(tiles[0])); ++i) {
+        const long width = ((c1 + 15) / 16 - a.tileN0) * 16L;
+        const long blocks = ((M + tiles[i].bm - 1) / tiles[i].bm) * ((width + tiles[i].bn - 1) / tiles[i].bn);
+        const long rounds = (blocks + device_cus() - 1) / device_cus();
+        const long c = rounds * ((long)KT * tiles[i].ns + 1500);
+        if (i == 0 || c < cost) cost = c, best = i;
     }
-    if (M > 128 && M <= 256) return launch_i8gemm_dma<64, 192, 2, 4, 8>(a, stream);
-    if (M > 256 && M <= 512) return launch_i8gemm_pp<128, 192, 2, 4, 6>(a, stream);
-    if (M <= 64) return launch_i8gemm<4, 1, 1, 2, 4, 4>(a, stream);
-    if (M <= 128) return launch_i8gemm_lds<128, 64, 2, 2, 4>(a, stream);
-    return launch_i8gemm_big<128, 192, 4, 2>(a, stream);
+    switch (best) {
+    case 0: return launch_i8gemm_roles<64, 16, 4, 1, 4, 4, 7>(a, stream);
+    case 1: return launch_i8gemm_roles<64, 32, 4, 1, 4, 2, 9>(a, stream);
+    case 2: return launch_i8gemm_roles<32, 48, 2, 1, 4, 4, 6>(a, stream);
+    case 3: return launch_i8gemm_roles<64, 48, 4, 1, 4, 2, 8>(a, stream);
+    case 4: return launch_i8gemm_roles<128, 32, 4, 1, 4, 2, 7>(a, stream);
+    case 5: return launch_i8gemm_roles<64, 64, 2, 2, 4, 2, 9>(a, stream);
+    case 6: return launch_i8gemm_roles<128, 48, 4, 1, 4, 2, 7>(a, stream);
+    case 7: return launch_i8gemm_roles<128, 64, 4, 2, 4, 2, 6>(a, stream);
+    case 8: return launch_i8gemm_roles<128, 96, 4, 2, 4, 1, 10>(a, stream);
+    case 9: return launch_i8gemm_roles<128, 128, 2, 4, 4, 1, 9>(a, stream);
+    case 10: return launch_i8gemm_roles<128, 192, 2, 4, 4, 1, 8>(a, stream);
+    }
+    return launch_i8gemm_pp<256, 256, 4, 2, 5>(a, stream);
 }
 
 template <int MODE, bool ROT>
@@ -1314,11 +1088,17 @@ int lm_i8_act(const float *x, long stride, int rows, int K, bool norm, float eps
 // columns into y[M][N/2]; y rows are y_stride floats apart. K % 64 == 0.
 // The batched pass's int8 GEMM over columns [a.c0, a.c1) in 256 x BN tiles.
 template <int BN>
-static int lm_i8_mm_tiles(int epi, const I8GemmArgs &a, hipStream_t stream) {
-    constexpr int NS = BN == 256 ? 5 : 6;
-    if (epi == 0) return launch_i8gemm_pp<256, BN, 4, 2, NS, true, I8_EPI_STORE>(a, stream);
-    if (epi == 1) return launch_i8gemm_pp<256, BN, 4, 2, NS, true, I8_EPI_ADD>(a, stream);
-    return launch_i8gemm_pp<256, BN, 4, 2, NS, true, I8_EPI_SWIGLU>(a, stream);
+static int lm_i8_mm_rows(int epi, const I8GemmArgs &a, hipStream_t stream) {
+    if (epi == 0) return launch_i8gemm_rows<BN, I8_EPI_STORE>(a, stream);
+    if (epi == 1) return launch_i8gemm_rows<BN, I8_EPI_ADD>(a, stream);
+    return launch_i8gemm_rows<BN, I8_EPI_SWIGLU>(a, stream);
+}
+
+template <int BM, int BN, int WGM, int WGN, int NP, int SB, int NS>
+static int lm_i8_mm_roles(int epi, const I8GemmArgs &a, hipStream_t stream) {
+    if (epi == 0) return launch_i8gemm_roles<BM, BN, WGM, WGN, NP, SB, NS, true, I8_EPI_STORE>(a, stream);
+    if (epi == 1) return launch_i8gemm_roles<BM, BN, WGM, WGN, NP, SB, NS, true, I8_EPI_ADD>(a, stream);
+    return launch_i8gemm_roles<BM, BN, WGM, WGN, NP, SB, NS, true, I8_EPI_SWIGLU>(a, stream);
 }
 
 int lm_i8_mm(int epi, const int8_t *act, const float *a_scale, const int8_t *codes, const float *w_scale, float *y,
@@ -1339,25 +1119,46 @@ int lm_i8_mm(int epi, const int8_t *act, const float *a_scale, const int8_t *cod
     a.c0 = 0;
     a.c1 = N;
     a.tileN0 = 0;
-    // 256 x 256 tiles on direct-to-LDS loads, the weights gathered from their
-    // rows. Measured on MI355X at M = 4096 (Qwen3-8B's projections, store
-    // epilogue) against the register-staged big-tile kernel on row-major
-    // operands: QKV 152 -> 141 us, gate/up 527 -> 479, down 207 -> 187; the
-    // ping-pong schedule with a 5-stage ring then took the pass 1.5% lower.
-    // A grid that is not whole rounds of the chip takes 256 x 256 tiles on the
-    // columns that fill whole rounds and 256 x 128 tiles (6-stage ring) on the
-    // rest (Qwen3-8B QKV at 4096 rows: 120.7 -> 72.2 + 47.5 us in a kernel
-    // trace, 143.7 -> 135.9 us with its activation pack timed by events).
-    const long full = whole_round_cols256((M + 255) / 256, (N + 255) / 256);
-    if (full > 0) {
-        I8GemmArgs b = a;
-        b.c1 = (int)(full * 256);
-        GPHQ_TRY(lm_i8_mm_tiles<256>(epi, b, stream));
-        a.c0 = b.c1;
-        a.tileN0 = a.c0 / 16;
-        return lm_i8_mm_tiles<128>(epi, a, stream);
+    // The tile with the least rounds of the chip x (K steps x time per step +
+    // fill and stores), as in i8gemm_launch; nanoseconds per 64-deep step
+    // measured on MI355X, K = 1024 to 12288. Columns past whole rounds of 256 x
+    // 256 tiles may take 256 x 128 ones. With their activation packs, rows 4 /
+    // 50 / 300 / 1500: Qwen3-8B down 128 / 130 / 136 / 163 us in 256-row tiles,
+    // 30.8 / 37.9 / 65.9 / 129 with this; O 47 / 48 / 53 / 68, 12.0 / 15.0 /
+    // 26.1 / 57.6; gate/up 52 / 60 / 72 / 199, 31 / 33 / 65 / 199.
+    struct Tile {
+        int bm, bn, ns, perCu;
+    };
+    static constexpr Tile tiles[] = {{16, 16, 118, 2},   {64, 32, 150, 1},   {64, 64, 207, 1},  {128, 64, 266, 1},
+                                     {128, 128, 385, 1}, {256, 128, 470, 1}, {256, 256, 700, 1}};
+    constexpr int kWide = 6, kSplit = 7;
+    auto time = [&](const Tile &t, long width) {
+        const long blocks = ((M + t.bm - 1L) / t.bm) * ((width + t.bn - 1) / t.bn), at_once = (long)device_cus() * t.perCu;
+        return (blocks + at_once - 1) / at_once * ((long)a.KT * t.ns + 1500);
+    };
+    int best = 0;
+    long cost = time(tiles[0], N);
+    for (int i = 1; i <= kWide; ++i) {
+        const long c = time(tiles[i], N);
+        if (c < cost) cost = c, best = i;
     }
-    return lm_i8_mm_tiles<256>(epi, a, stream);
+    const long full = whole_round_cols256((M + 255) / 256, (N + 255) / 256);
+    if (full > 0 && time(tiles[kWide], full * 256) + time(tiles[kWide - 1], N - full * 256) < cost) best = kSplit;
+    switch (best) {
+    case 0: return lm_i8_mm_roles<16, 16, 1, 1, 2, 4, 8>(epi, a, stream);
+    case 1: return lm_i8_mm_roles<64, 32, 4, 1, 4, 2, 9>(epi, a, stream);
+    case 2: return lm_i8_mm_roles<64, 64, 2, 2, 4, 2, 9>(epi, a, stream);
+    case 3: return lm_i8_mm_roles<128, 64, 4, 2, 4, 2, 6>(epi, a, stream);
+    case 4: return lm_i8_mm_roles<128, 128, 2, 4, 4, 1, 9>(epi, a, stream);
+    case 5: return lm_i8_mm_rows<128>(epi, a, stream);
+    case kWide: return lm_i8_mm_rows<256>(epi, a, stream);
+    }
+    I8GemmArgs b = a;
+    b.c1 = (int)(full * 256);
+    GPHQ_TRY(lm_i8_mm_rows<256>(epi, b, stream));
+    a.c0 = b.c1;
+    a.tileN0 = a.c0 / 16;
+    return lm_i8_mm_rows<128>(epi, a, stream);
 }
 
 int i8_pack_tiles(const int8_t *src, int8_t *dst, int rows, int K, int row0, int kt, hipStream_t stream) {

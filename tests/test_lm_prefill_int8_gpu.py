@@ -125,6 +125,38 @@ def test_project_int8_residual_add_bit_exact(geom, proj, rows):
     assert np.array_equal(got.view(np.uint32), want.astype(np.float32).view(np.uint32))
 
 
+@pytest.mark.parametrize("rows", [16, 17, 65, 120, 129, 700, 1030])
+def test_project_int8_tile_shapes_bit_exact(rows):
+    """Row counts on both sides of the tile shapes' edges."""
+    test_project_int8_residual_add_bit_exact(lc.SMALL_06B, 3, rows)
+
+
+@pytest.mark.parametrize("rows", [40, 400, 1500, 3000])
+def test_project_int8_odd_steps_bit_exact(rows):
+    """K = 1088 = 17 steps of 64: the whole-line loads' last piece is half a line
+    (3000 rows: 256 x 256 tiles). Sums from a float64 product of the codes."""
+    import torch
+
+    geom = lo.Geometry(hidden=4096, layers=1, heads=32, kv_heads=8, head_dim=128, inter=1088, vocab=256, max_pos=64)
+    model, _, lm = setup(geom, lo.FMT_Q8, seed=8)
+    W, sw, n, k = _layer_weights(model, 3)
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    y0 = rng.standard_normal((rows, n)).astype(np.float32)
+    ws = gphq.Prefill(lm, rows)
+    ws.set_arith(gphq.PASS_INT8)
+    xd, yd = torch.from_numpy(x).cuda(), torch.from_numpy(y0).cuda()
+    print(f"project int8 proj=3 rows={rows} k={k} n={n}", flush=True)
+    ws.project(0, 3, xd, rows, yd)
+    got = yd.cpu().numpy()
+    rot = lo.rotation(k)
+    xin = np.stack([orc.rotation_apply_f32(row, rot) for row in x])
+    qa, sa, _ = orc.i8_pack_rows(xin, rows, k)
+    sums = (torch.from_numpy(qa.astype(np.float64)).cuda() @ torch.from_numpy(W.astype(np.float64)).cuda().T).cpu().numpy()
+    v = (sums.astype(np.float32) * sw[None, :]) * sa[:, None]
+    assert np.array_equal(got.view(np.uint32), (y0 + v).astype(np.float32).view(np.uint32))
+
+
 @pytest.mark.parametrize("proj", [0, 2])
 @pytest.mark.parametrize("rows", [1, 64, 257])
 def test_project_int8_normalized_inputs(proj, rows):

@@ -123,6 +123,27 @@ def test_config2_shapes_bit_exact(m):
     del torch
 
 
+@pytest.mark.parametrize("m,n", [(17, 50), (31, 12200), (50, 4500), (64, 9000), (100, 5000), (110, 7800), (129, 3000),
+                                 (130, 9300), (190, 12240), (257, 20000), (300, 9000), (520, 12300), (1030, 8200),
+                                 (1100, 16000)])
+@pytest.mark.parametrize("k", [64, 65, 190, 256, 735])
+def test_tile_shapes_and_last_steps_bit_exact(m, n, k):
+    """Every tile shape of the dispatch over 1, 2, 3, 4 and 12 K-steps (fewer
+    than the ring's stages, and last stages cut short), partial row and column
+    tiles: exact integer sums from a float64 product of the codes."""
+    rng = np.random.default_rng(m + n + k)
+    q = rng.integers(-127, 128, k * n).astype(np.int8)
+    scales = (np.abs(rng.standard_normal(n)) * 0.01).astype(np.float32)
+    w = gphq.WeightsI8(k, n)
+    w.pack(q, scales)
+    x = rng.standard_normal(m * k).astype(np.float32)
+    got, _ = run_gpu(x, m, k, w, n)
+    qa, rs, _ = orc.i8_pack_rows(x, m, k)
+    acc = host(dev(qa.astype(np.float64)) @ dev(q.reshape(n, k).astype(np.float64)).T)
+    want = (acc.astype(np.float32) * scales[None, :]).astype(np.float32) * rs[:, None]
+    assert np.array_equal(got.reshape(m, n).view(np.uint32), want.astype(np.float32).view(np.uint32))
+
+
 def test_golden_tile():
     g = np.load(os.path.join(GOLDEN, "i8_tile.npz"))
     rows, k = g["x"].shape
