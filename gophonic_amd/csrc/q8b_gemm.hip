@@ -24,51 +24,49 @@ typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// One thread per (row, 32-value block): scale = max/127 and inverse = 127/max
-// (both 0 unless 0 < max < inf, int8.go:106-119), codes RNE(x * inverse)
-// saturated to int8 (int8.go:163-168; a NaN product gives 0).
-__global__ __launch_bounds__(256) void q8b_quantize_kernel(const float *__restrict__ x, int rows, int k, long stride,
-                                                           int8_t *__restrict__ q, float *__restrict__ d) {
+// Scale = max/127 and inverse = 127/max per (row, 32-value block), both 0
+// unless 0 < max < inf (int8.go:106-119), codes RNE(x * inverse) saturated to
+// int8 (int8.go:163-168). Latency-bound: eight lanes share a block, one float4
+// each, so a wavefront reads 1 KiB in one load and all of it is in flight at
+// once (one lane per block read lines in eight passes, 128 bytes apart). The
+// maximum is taken over the bits of |x|, where infinities and NaN order above
+// every finite value. A grid of at most kQuantGrid blocks walks (row, 1024
+// columns) chunks.
+constexpr long kQuantGrid = 1 << 20;
+
+__global__ __launch_bounds__(256) void q8b_quantize_kernel(const float *__restrict__ x, long chunks, int perRow, int k,
+                                                           long stride, int8_t *__restrict__ q,
+                                                           float *__restrict__ d) {
     const int kb = k >> 5;
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long)rows * kb) return;
-    const int r = (int)(idx / kb), b = (int)(idx - (long)r * kb);
-    const float4 *src = (const float4 *)(x + r * stride + b * 32);
-    float v[32];
-    float mx = 0.0f;
-    bool nan = false;
+    for (long ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
+        const long r = ch / perRow;
+        const int c4 = (int)(ch - r * perRow) * 256 + (int)threadIdx.x;  // float4 of the row
+        if (c4 >= kb * 8) continue;  // whole groups of eight lanes: kb * 8 is a multiple of 8
+        const float4 f = *(const float4 *)(x + r * stride + (long)c4 * 4);
+        const float v[4] = {f.x, f.y, f.z, f.w};
+        uint32_t mb = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float4 f = src[i];
-        v[4 * i] = f.x, v[4 * i + 1] = f.y, v[4 * i + 2] = f.z, v[4 * i + 3] = f.w;
-    }
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        nan |= v[i] != v[i];
-        mx = fmaxf(mx, fabsf(v[i]));
-    }
-    float s = 0.0f, inv = 0.0f;
-    if (!nan && mx > 0.0f && mx != INFINITY) {
-        s = __fdiv_rn(mx, 127.0f);
-        inv = __fdiv_rn(127.0f, mx);
-    }
-    d[idx] = s;
-    int32_t packed[8];
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
+        for (int i = 0; i < 4; ++i) mb = max(mb, __float_as_uint(v[i]) & 0x7fffffffu);
+        mb = max(mb, (uint32_t)__builtin_amdgcn_mov_dpp((int)mb, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+        mb = max(mb, (uint32_t)__builtin_amdgcn_mov_dpp((int)mb, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+        mb = max(mb, (uint32_t)__builtin_amdgcn_mov_dpp((int)mb, 0x141, 0xF, 0xF, true));  // row_half_mirror
+        float s = 0.0f, inv = 0.0f;
+        if (mb > 0 && mb < 0x7f800000u) {
+            const float mx = __uint_as_float(mb);
+            s = __fdiv_rn(mx, 127.0f);
+            inv = __fdiv_rn(127.0f, mx);
+        }
         uint32_t word = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float p = __fmul_rn(v[4 * w + j], inv);
+            const float p = __fmul_rn(v[j], inv);
             float c = p != p ? 0.0f : rintf(p);
             c = fminf(127.0f, fmaxf(-128.0f, c));
             word |= (uint32_t)(uint8_t)(int8_t)(int)c << (8 * j);
         }
-        packed[w] = (int32_t)word;
+        *(uint32_t *)(q + r * k + (long)c4 * 4) = word;
+        if ((c4 & 7) == 0) d[r * kb + (c4 >> 3)] = s;
     }
-    int32_t *dst = (int32_t *)(q + (long)r * k + b * 32);
-    *(i32x4 *)dst = i32x4{packed[0], packed[1], packed[2], packed[3]};
-    *(i32x4 *)(dst + 4) = i32x4{packed[4], packed[5], packed[6], packed[7]};
 }
 
 struct Q8bArgs {
@@ -299,6 +297,162 @@ __global__ __launch_bounds__(64 * WGM * WGN) void q8b_gemm_kernel(const Q8bArgs 
         }
 }
 
+// BM x BN output tiles, WGM x WGN wavefronts of 16 TI x 16 TJ outputs, one
+// v_mfma_i32_16x16x32_i8 per 16 x 16 outputs and 32-value block. The
+// scale-accumulate is three VALU instructions per output and block (128 x
+// 12288 outputs at K = 4096: 15 us if every SIMD had the same share), so the
+// tile decides how evenly the SIMDs share it: 32 x 32 MFMAs in 64 x 64 tiles gave
+// half the CUs twice the others' work there, 64 x 96 tiles of these give every
+// SIMD six 16 x 16 tiles (44.6 -> 36.8 us).
+// Codes pass through LDS in rows of KSB * 32 bytes, 16-byte chunks
+// XOR-swizzled (swz) so that the 8-byte fragment reads of 16 rows at one chunk
+// cover all 64 banks; weight scales stay [row][block] (one float4 read per
+// four blocks), activation scales [block][row]. Two LDS buffers; the next
+// step's loads are issued before a step's products and stored after them.
+// Rows past m or n and chunks past k repeat the last one: their rows are not
+// stored and their blocks are skipped, and so are 16-row tiles past m. The
+// chain per output is in block order, the same bits as the other kernels.
+template <int TI, int TJ, int WGM, int WGN, int KSB>
+__global__ __launch_bounds__(64 * WGM * WGN) void q8b_tile_kernel(const Q8bArgs a) {
+    constexpr int NT = 64 * WGM * WGN, BM = 16 * TI * WGM, BN = 16 * TJ * WGN;
+    constexpr int CH = 2 * KSB, UNITS = (BM + BN) * CH, LU = (UNITS + NT - 1) / NT;
+    constexpr int SU = (BM + BN) * (KSB / 4), SL = (SU + NT - 1) / NT, SBS = KSB + 4;
+    static_assert((KSB == 4 || KSB == 8) && BM * CH % 64 == 0, "swizzle; whole wavefronts load one operand");
+    __shared__ __align__(16) int8_t cs[2][(BM + BN) * KSB * 32];
+    __shared__ __align__(16) float Sa[2][KSB][BM];
+    __shared__ __align__(16) float Sb[2][BN][SBS];
+    int bm, bn;
+    tile_order(blockIdx.x, a.gridM, a.gridN, bm, bn);
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wv / WGN, wn = wv % WGN, m0 = bm * BM, n0 = bn * BN;
+    const int kb = a.k >> 5, steps = (kb + KSB - 1) / KSB;
+    auto swz = [](int row, int c) { return KSB == 8 ? c ^ (row & 15) : c ^ ((row >> 1) & 7); };
+    // Unit u = i * NT + t: 16-byte chunk u % CH of row u / CH, A's rows first.
+    const int8_t *src[LU];
+    int dst[LU];
+#pragma unroll
+    for (int i = 0; i < LU; ++i) {
+        const int u = min(i * NT + t, UNITS - 1), row = u / CH, ch = u % CH;
+        src[i] = row < BM ? a.qa + (size_t)min(m0 + row, a.m - 1) * a.k : a.qw + (size_t)min(n0 + row - BM, a.n - 1) * a.k;
+        dst[i] = row * (KSB * 32) + swz(row, ch) * 16;
+    }
+    const float *ssrc[SL];
+#pragma unroll
+    for (int i = 0; i < SL; ++i) {
+        const int row = min(i * NT + t, SU - 1) / (KSB / 4);
+        ssrc[i] = row < BM ? a.da + (size_t)min(m0 + row, a.m - 1) * kb : a.dw + (size_t)min(n0 + row - BM, a.n - 1) * kb;
+    }
+    i32x4 cr[LU];
+    f32x4 sr[SL];
+    auto gload = [&](int st) {
+#pragma unroll
+        for (int i = 0; i < LU; ++i) {
+            const int u = min(i * NT + t, UNITS - 1);
+            cr[i] = *(const i32x4 *)(src[i] + min(st * (KSB * 32) + (u % CH) * 16, a.k - 16));
+        }
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+            const int b0 = st * KSB + min(i * NT + t, SU - 1) % (KSB / 4) * 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sr[i][e] = ssrc[i][min(b0 + e, kb - 1)];
+        }
+    };
+    auto lstore = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LU; ++i)
+            if ((i + 1) * NT <= UNITS || i * NT + t < UNITS) *(i32x4 *)&cs[buf][dst[i]] = cr[i];
+#pragma unroll
+        for (int i = 0; i < SL; ++i) {
+            const int v = i * NT + t;
+            if (v >= SU) continue;
+            const int quad = v % (KSB / 4), row = v / (KSB / 4);
+            if (row < BM) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) Sa[buf][quad * 4 + e][row] = sr[i][e];
+            } else {
+                *(f32x4 *)&Sb[buf][row - BM][quad * 4] = sr[i];
+            }
+        }
+    };
+    const int c = lane & 15, g = lane >> 4;
+    f32x4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4{};
+    int ti = 0;  // the wavefront's 16-row tiles that hold rows of the matrix
+#pragma unroll
+    for (int i = 0; i < TI; ++i) ti += m0 + (wm * TI + i) * 16 < a.m;
+    gload(0);
+    lstore(0);
+    __syncthreads();
+    for (int st = 0; st < steps; ++st) {
+        const int cur = st & 1, nb = min(KSB, kb - st * KSB);
+        if (st + 1 < steps) gload(st + 1);
+        auto frag = [&](int row, int b) {
+            return *(const long *)&cs[cur][row * (KSB * 32) + swz(row, 2 * b + (g >> 1)) * 16 + (g & 1) * 8];
+        };
+        // Block b + 1's MFMAs are issued before block b's scale-accumulates.
+        auto issue = [&](int b, i32x4(&d)[TI][TJ]) {
+            long av[TI], bv[TJ];
+#pragma unroll
+            for (int i = 0; i < TI; ++i) av[i] = frag((wm * TI + i) * 16 + c, b);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) bv[j] = frag(BM + (wn * TJ + j) * 16 + c, b);
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j)
+                    d[i][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i], bv[j], i32x4{}, 0, 0, 0);
+        };
+        f32x4 sb[TJ];
+        auto apply = [&](int b, const i32x4(&d)[TI][TJ]) {
+            if (b % 4 == 0)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) sb[j] = *(const f32x4 *)&Sb[cur][(wn * TJ + j) * 16 + c][b];
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+                const f32x4 sa = *(const f32x4 *)&Sa[cur][b][(wm * TI + i) * 16 + 4 * g];
+#pragma unroll
+                for (int j = 0; j < TJ; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i][j][e] = __builtin_fmaf((float)d[i][j][e], __fmul_rn(sa[e], sb[j][b % 4]), acc[i][j][e]);
+            }
+        };
+        i32x4 d[2][TI][TJ];
+        if (ti > 0 && nb == KSB) {
+            issue(0, d[0]);
+#pragma unroll
+            for (int b = 0; b < KSB; ++b) {
+                if (b + 1 < KSB) issue(b + 1, d[(b + 1) & 1]);
+                apply(b, d[b & 1]);
+            }
+        } else if (ti > 0) {
+#pragma unroll
+            for (int b = 0; b < KSB; ++b)
+                if (b < nb) {
+                    issue(b, d[0]);
+                    apply(b, d[0]);
+                }
+        }
+        if (st + 1 < steps) lstore(cur ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int col = n0 + (wn * TJ + j) * 16 + c;
+            if (col >= a.n) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = m0 + (wm * TI + i) * 16 + 4 * g + e;
+                if (row < a.m) a.y[(size_t)row * a.n + col] = acc[i][j][e];
+            }
+        }
+}
+
 // M <= 16 * TI: one wavefront (and block) per 16 weight rows, all
 // activation rows in TI tiles of 16. A step is 128 bytes of K (four
 // blocks): the wavefront loads its 16 weight rows and 16 * TI activation
@@ -515,12 +669,6 @@ int go_small(const Q8bArgs &a, hipStream_t st) {
     return launch_status();
 }
 
-// Ring depth 8 steps for one activation tile, 4 for two (registers).
-template <int TI>
-int launch_small(const Q8bArgs &a, hipStream_t st) {
-    return go_small<TI, TI == 1 ? 8 : 4>(a, st);
-}
-
 template <int BM, int BN, int WGM, int WGN, int KSB>
 int launch_q8b(Q8bArgs a, hipStream_t st) {
     a.gridM = (a.m + BM - 1) / BM;
@@ -528,6 +676,51 @@ int launch_q8b(Q8bArgs a, hipStream_t st) {
     hipLaunchKernelGGL((q8b_gemm_kernel<BM, BN, WGM, WGN, KSB>), dim3((unsigned)(a.gridM * a.gridN)),
                        dim3(64 * WGM * WGN), 0, st, a);
     return launch_status();
+}
+
+template <int TI, int TJ, int WGM, int WGN, int KSB>
+int launch_tile(Q8bArgs a, hipStream_t st) {
+    constexpr int BM = 16 * TI * WGM, BN = 16 * TJ * WGN;
+    a.gridM = (a.m + BM - 1) / BM;
+    a.gridN = (a.n + BN - 1) / BN;
+    hipLaunchKernelGGL((q8b_tile_kernel<TI, TJ, WGM, WGN, KSB>), dim3((unsigned)(a.gridM * a.gridN)),
+                       dim3(64 * WGM * WGN), 0, st, a);
+    return launch_status();
+}
+
+// The tile with the least time at rounds r = ceil(blocks / 256 CUs), each tile
+// with its least time (one block alone on a CU waits for its own loads), a
+// fixed time and a time per round, in tenths of a microsecond at K = 4096,
+// fitted to 33-512 rows at N = 600, 1000, 3396 and 12288 (K changes all
+// of them alike). Measured at K = 4096 on MI355X, 32 x 32 / 64 x 48 / 64 x 64 /
+// 64 x 96 / 128 x 192: 64 rows, N = 3396 (one round of each) 15.8 / 31.3 /
+// 38.0 / 35.2 / - us; N = 12288, 64 rows 24.4 / 32.1 / 38.2 / 36.2 / -, 128 rows
+// 43.6 / 39.2 / 44.6 / 36.8 / -, 160 rows 56.6 / 47.9 / 55.5 / 66.6 / -, 256
+// rows 81.6 / 63.2 / 60.6 / 73.7 / 87.3, 512 rows 159 / 118 / 114 / 137 / 95.
+// Small tiles win while several of them share a CU and hide each other's loads;
+// large ones once LDS reads and not latency set the time. 32 rows, N = 12288 /
+// 3396 and K = 8192, N = 600: 27.3 / 21.4 / 40.3 us with one wavefront per 16
+// weight rows (q8b_small_kernel, kept for up to 16 rows: 18.9 / 12.8 / 22.0 us),
+// 20.2 / 15.1 / 26.3 us in 32 x 32 tiles.
+enum Tile { kTile32x32, kTile64x48, kTile64x64, kTile64x96, kTile128x192 };
+
+Tile tile_for(int64_t m, int64_t n) {
+    static constexpr struct {
+        int bm, bn, least, fixed, round;
+    } kTiles[] = {{32, 32, 160, 40, 66},
+                  {64, 48, 320, 100, 134},
+                  {64, 64, 380, 100, 170},
+                  {64, 96, 345, 20, 345},
+                  {128, 192, 870, 0, 920}};
+    int best = 0;
+    int64_t shortest = INT64_MAX;
+    for (int i = 0; i < 5; ++i) {
+        const int64_t blocks = ((m + kTiles[i].bm - 1) / kTiles[i].bm) * ((n + kTiles[i].bn - 1) / kTiles[i].bn);
+        const int64_t t = kTiles[i].fixed + (blocks + 255) / 256 * kTiles[i].round;
+        const int64_t time = t < kTiles[i].least ? kTiles[i].least : t;
+        if (time < shortest) shortest = time, best = i;
+    }
+    return (Tile)best;
 }
 
 }  // namespace
@@ -540,9 +733,10 @@ int gphq_q8b_quantize(const float *x_dev, int64_t rows, int64_t k, int64_t x_str
         return GPHQ_ERR_DIMENSIONS;
     if (rows == 0 || k == 0) return GPHQ_OK;
     if (!x_dev || !q_dev || !d_dev) return GPHQ_ERR_DIMENSIONS;
-    const long items = (long)rows * (k / 32);
-    hipLaunchKernelGGL(q8b_quantize_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                       x_dev, (int)rows, (int)k, (long)x_stride, q_dev, d_dev);
+    const int perRow = (int)((k / 4 + 255) / 256);
+    const long chunks = (long)rows * perRow;
+    hipLaunchKernelGGL(q8b_quantize_kernel, dim3((unsigned)(chunks < kQuantGrid ? chunks : kQuantGrid)), dim3(256), 0,
+                       (hipStream_t)stream, x_dev, chunks, perRow, (int)k, (long)x_stride, q_dev, d_dev);
     return launch_status();
 }
 
@@ -555,15 +749,19 @@ int gphq_q8b_gemm(const int8_t *qa_dev, const float *da_dev, const int8_t *qw_de
     if (k == 0) return fill_f32(y_dev, (size_t)m * n, 0.0f, (hipStream_t)stream);
     Q8bArgs a{qa_dev, da_dev, qw_dev, dw_dev, y_dev, (int)m, (int)k, (int)n, 0, 0};
     hipStream_t st = (hipStream_t)stream;
-    // Shapes measured on MI355X at K = 4096, N = 12288: from M = 256,
-    // 128 x 192 tiles of eight wavefronts (one per CU at M = 512); from
-    // M = 33, 64 x 64 tiles with 256-byte K steps; one row at K = 2048, 4096,
-    // 8192 or 12288, whole weight rows streamed per wavefront; otherwise up
-    // to 32 rows (k a multiple of 128), one wavefront per 16 weight rows with
-    // a ring of steps in flight.
-    if (m >= 256) return launch_q8b<128, 192, 4, 2, 4>(a, st);
-    if (m > 32) return launch_q8b<64, 64, 2, 2, 8>(a, st);
-    if (k % 128) return launch_q8b<64, 64, 2, 2, 4>(a, st);
+    // Up to 16 rows with k a multiple of 128: one row at K = 2048, 4096, 8192 or
+    // 12288 streams whole weight rows per wavefront, the others one wavefront
+    // per 16 weight rows with a ring of steps in flight. Everything else takes
+    // the tile of tile_for.
+    if (m > 16 || k % 128) {
+        switch (tile_for(m, n)) {
+        case kTile32x32: return launch_tile<1, 1, 2, 2, 8>(a, st);
+        case kTile64x48: return launch_tile<1, 3, 4, 1, 4>(a, st);
+        case kTile64x64: return launch_tile<2, 2, 2, 2, 4>(a, st);
+        case kTile64x96: return launch_tile<1, 3, 4, 2, 8>(a, st);
+        case kTile128x192: return launch_q8b<128, 192, 4, 2, 4>(a, st);
+        }
+    }
     if (m == 1) {
         switch (k) {
         case 2048: return go_gemv<2>(a, st);
@@ -572,8 +770,7 @@ int gphq_q8b_gemm(const int8_t *qa_dev, const float *da_dev, const int8_t *qw_de
         case 12288: return go_gemv<12>(a, st);
         }
     }
-    if (m > 16) return launch_small<2>(a, st);
-    return launch_small<1>(a, st);
+    return go_small<1, 8>(a, st);  // a ring of eight steps in flight
 }
 
 }  // extern "C"

@@ -61,6 +61,30 @@ def test_gemm_bit_exact(m, k, n):
     assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,k,n", [(70, 288, 530), (150, 160, 12200), (250, 160, 12200), (100, 160, 12200),
+                                   (500, 160, 12200), (33, 32, 33), (3, 32, 1)])
+def test_gemm_tiles_bit_exact(m, k, n):
+    # Each tile of the size rule (32 x 32, 64 x 48, 64 x 64, 64 x 96, 128 x 192, in this order) with rows, columns
+    # and K past whole tiles and steps, then the smallest calls: the bits of the oracle's block-ordered chain.
+    test_gemm_bit_exact(m, k, n)
+
+
+def test_quantize_ragged_rows_and_chunks():
+    # A row stride past k, k past whole 1024-column chunks, and NaN, infinite and zero blocks at a chunk's edge.
+    import torch
+
+    rng = np.random.default_rng(3)
+    rows, k, stride = 5, 1056, 1060
+    x = rng.standard_normal((rows, stride)).astype(np.float32)
+    x[0, 1023], x[1, 1024], x[2, 1024:1056], x[3, 1055] = np.nan, -np.inf, 0.0, 1e30
+    q = torch.empty((rows, k), dtype=torch.int8, device="cuda")
+    d = torch.empty((rows, k // 32), dtype=torch.float32, device="cuda")
+    gphq.q8b_quantize(dev(x), rows, k, q, d, x_stride=stride)
+    wq, wd = orc.q8b_quantize(np.ascontiguousarray(x[:, :k]), rows, k)
+    assert np.array_equal(q.cpu().numpy(), wq)
+    assert np.array_equal(d.cpu().numpy().view(np.uint32), wd.view(np.uint32))
+
+
 @pytest.mark.parametrize("m", [1, 16, 128, 512])
 def test_config2_shape_rows_bit_exact(m):
     # Benchmark configuration 2 (K = 4096, N = 12288) at each bench M: sampled
