@@ -71,12 +71,12 @@ def oracle_out(x, rows, k, q, scales, n):
 SHAPES = [(1, 4, 1), (3, 7, 17), (12, 64, 64), (16, 257, 129), (12, 4096, 1024), (5, 12288, 64), (1, 32, 64),
           (1, 4096, 1024), (1, 12288, 200), (1, 96, 5), (17, 100, 33), (64, 640, 96), (100, 512, 300),
           (200, 1024, 520),
-          # the skinny kernel (17..256 rows, K a multiple of 256): one-stage K,
+          # 17..256 rows, K a multiple of 256: one-stage K,
           # column tiles past N in a block, two row blocks
           (24, 256, 200), (48, 256, 500), (130, 1024, 64), (256, 2048, 77), (33, 12288, 48),
-          # direct-to-LDS big tiles (129..512 rows), K not a multiple of 256
+          # 129..512 rows, K not a multiple of 256
           (300, 640, 260), (512, 192, 200), (140, 64, 40),
-          # K not a multiple of 256 from 65 rows (LDS kernel) and past 512 rows (big tiles)
+          # K not a multiple of 256 from 65 rows and past 512 rows
           (100, 640, 200), (600, 320, 130)]
 
 
