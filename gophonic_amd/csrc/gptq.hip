@@ -308,7 +308,10 @@ __device__ __forceinline__ void chol16_steps(double (&a)[16], double (&w)[4], in
         double d = row_bcast<J>(a[J]);
         const bool positive = d > 0.0;
         fail = fail || !positive;
-        d = positive ? d : 1.0;
+        // An infinite pivot (an overflowed Gram matrix) is the reference's
+        // sqrt(Inf): Inf on the diagonal, zeros below it and in the inverse.
+        // Bounded here it gives the same float32 values without Inf * 0 below.
+        d = positive ? fmin(d, 1e300) : 1.0;
         // sqrt(d) and its reciprocal from the hardware's estimate, two Goldschmidt steps.
         double r = __builtin_amdgcn_rsq(d), piv = d * r, hr = 0.5 * r;
 #pragma unroll
@@ -324,7 +327,7 @@ __device__ __forceinline__ void chol16_steps(double (&a)[16], double (&w)[4], in
         const double li = i > J ? l : 0.0;
         chol16_row<J, J + 1>(a, l, li);
         // The reciprocal of the stored pivot; row J of the inverse is final.
-        const double ljj = row_bcast<J>(l);
+        const double ljj = fmin(row_bcast<J>(l), 1e150);
 #pragma unroll
         for (int n = 0; n < 2; ++n) r = fma(r, fma(-ljj, r, 1.0), r);
         const double lr = li * r;

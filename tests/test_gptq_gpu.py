@@ -101,6 +101,28 @@ def test_factor_at_panel_edges(k):
     assert np.abs(h @ (u64.T @ u64) - np.eye(k)).max() <= 1e-4
 
 
+@pytest.mark.parametrize("k", [1, 2, 20, 64, 65, 80])
+def test_factor_with_an_infinite_pivot(k):
+    """choleskyLower refuses a pivot only when !(d > 0) (gptq_linalg.go:73-93): sqrt(+Inf) is a pivot, its column
+    of the factor and of the inverse zero. A Gram matrix that overflows (all pivots infinite once damped) factors to
+    zeros, and a diagonal entry that overflows only when damped leaves the other channels their own factor."""
+    rng = np.random.default_rng(k)
+    for at in {0, k // 2, k - 1}:
+        x = rng.standard_normal((k + 5, k))
+        x[:, at] = 1e20 * np.sign(x[:, at])
+        u, dead = factor(x.astype(np.float32))
+        assert not dead.any() and not u.any()
+        x = rng.standard_normal((k + 5, k))
+        x[:, at] = 0
+        x[0, at] = 1.8446e19  # its square + 0.01 / k of it is past the float32 range
+        u, dead = factor(x.astype(np.float32))
+        assert not dead.any() and not u[at].any() and not u[:, at].any()
+        rest = np.arange(k) != at
+        add = 0.01 * float(np.float32(1.8446e19)) ** 2 / k  # dwarfs the other channels' own sums
+        assert np.allclose(np.diag(u)[rest], add ** -0.5, rtol=1e-5, atol=0)
+        assert np.array_equal(u, np.triu(u)) and np.isfinite(u).all()
+
+
 def test_factor_rejects_non_finite_hessian():
     import torch
 
