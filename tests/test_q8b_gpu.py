@@ -85,6 +85,23 @@ def test_quantize_ragged_rows_and_chunks():
     assert np.array_equal(d.cpu().numpy().view(np.uint32), wd.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,k,stride", [(1, 32, 32), (257, 32, 32), (4099, 32, 36), (1001, 96, 100),
+                                           (2049, 4096, 4096), (2050, 4096, 4100), (2100, 4000, 4004)])
+def test_quantize_row_lengths(rows, k, stride):
+    # Rows of one block, rows that share a wavefront and thread blocks that end inside a row, with and without gaps
+    # between rows, on both sides of the size from which a thread takes two pieces. Rows scaled apart.
+    import torch
+
+    rng = np.random.default_rng(rows + k)
+    x = rng.standard_normal((rows, stride)).astype(np.float32) * np.exp2(np.arange(rows) % 61 - 30)[:, None].astype(np.float32)
+    q = torch.empty((rows, k), dtype=torch.int8, device="cuda")
+    d = torch.empty((rows, k // 32), dtype=torch.float32, device="cuda")
+    gphq.q8b_quantize(dev(x), rows, k, q, d, x_stride=stride)
+    wq, wd = orc.q8b_quantize(np.ascontiguousarray(x[:, :k]), rows, k)
+    assert np.array_equal(q.cpu().numpy(), wq)
+    assert np.array_equal(d.cpu().numpy().view(np.uint32), wd.view(np.uint32))
+
+
 @pytest.mark.parametrize("m", [1, 16, 128, 512])
 def test_config2_shape_rows_bit_exact(m):
     # Benchmark configuration 2 (K = 4096, N = 12288) at each bench M: sampled
