@@ -10,13 +10,13 @@
 //     exact power of two 2^e (its max into [2^14, 2^15)) and splits it into
 //     FP16 hi + lo parts (x*2^e = hi + lo + r, |r| <= 2^-22 |x*2^e|), laid out
 //     as MFMA A fragments;
-//   * vecs_kernel widens each 32-value block of 16 weight rows to FP16 (int8
-//     and 4-bit codes are exact in FP16), runs v_mfma_f32_16x16x32_f16 on it
-//     (products exact in fp32), and folds the block result into fp32
-//     accumulators with the weight block scale and the activation block's
-//     2^-e: acc = fma(d*2^-e, C, acc), the per-block scaling of the qwen3lm
-//     kernels;
-//   * K is split over wavefronts; partial sums meet in LDS in slice order;
+//   * vecs_kernel, or vecd_kernel for small products (vecd_rows), widens each
+//     32-value block of 16 weight rows to FP16 (int8 and 4-bit codes are exact
+//     in FP16), runs v_mfma_f32_16x16x32_f16 on it (products exact in fp32),
+//     and folds the block result into fp32 accumulators with the weight block
+//     scale and the activation block's 2^-e: acc = fma(d*2^-e, C, acc), the
+//     per-block scaling of the qwen3lm kernels;
+//   * K is split over wavefronts; partial sums meet in LDS in a fixed order;
 //     y[v][n] = acc_hi + acc_lo (Q8: times the row scale; PRO_NORM: times
 //     1/sqrt(mean(x^2) + eps) from the prep pass's block sums of squares).
 // 8-bit formats with up to 16 vectors and K a multiple of 512 take
@@ -72,10 +72,9 @@ __host__ __device__ inline size_t vec_a_offset(int t, int kb, int KB, int lane) 
 }
 
 // ---- multi-vector GEMV with per-block activation scales ----------------------
-// The A tiles of V vectors: up to 8 vectors, one tile with hi and lo of vector
-// v in rows 2v and 2v + 1; up to 16, a hi tile and a lo tile with vector v in
-// row v (PAIR, half the result registers); more, the first kind, 8 vectors a
-// tile.
+// The A tiles of V vectors: 8 vectors a tile, hi and lo of vector v in rows 2v
+// and 2v + 1 (mod 16); for vecs_kernel from 9 to 16 vectors a hi tile and a lo
+// tile with vector v in row v (PAIR, half the result registers).
 __host__ __device__ inline bool vec_pair(int V) { return V > 8 && V <= 16; }
 
 // vec_prep_blocks_kernel: four threads per (vector v, 32-value block kb), 8
@@ -86,7 +85,7 @@ __host__ __device__ inline bool vec_pair(int V) { return V > 8 && V <= 16; }
 // for any vector count.
 __global__ __launch_bounds__(256) void vec_prep_blocks_kernel(const float *__restrict__ x, long stride, int V, int KB,
                                                               _Float16 *__restrict__ A, float *__restrict__ inv,
-                                                              float *__restrict__ ssq) {
+                                                              float *__restrict__ ssq, bool pair) {
     const long t4 = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int gq = (int)(t4 & 3);
     const long idx = min(t4 >> 2, (long)V * KB - 1);  // the last block's extra threads repeat its work
@@ -116,7 +115,6 @@ __global__ __launch_bounds__(256) void vec_prep_blocks_kernel(const float *__res
         hi[i] = h;
         lo[i] = (_Float16)(y - (float)h);
     }
-    const bool pair = vec_pair(V);
     const int th = pair ? 0 : v >> 3, tl = pair ? 1 : th;
     const int rh = pair ? v : (2 * v) & 15, rl = pair ? v : rh + 1;
     *(f16x8 *)(A + vec_a_offset(th, kb, KB, gq * 16 + rh)) = hi;
@@ -140,14 +138,167 @@ struct Vec2Args {
     float *part;  // K-split stationary path: [parts][V][N] partial sums
 };
 
+// Small products over prepared A fragments, operands straight from global
+// memory: each wavefront applies its A fragments to RT tiles of 16 weight rows, U blocks at a time. All U*RT*MT
+// MFMAs of a step are issued before their results are scaled and summed
+// (acc += d * 2^-e_v * C), which keeps the MFMA latency off the critical path.
+// VALU work per weight is the code conversion (v_perm + packed FP16
+// subtract). K is split over the SK wavefronts of the block; partial sums meet
+// in a fixed LDS tree, and PRO_NORM's sum of squares is read from the prep
+// pass's block sums in block order.
+template <int FMT, int MT, int SK, int RT, int U, int EPI, bool NORM>
+__global__ __launch_bounds__(64 * SK) void vecd_kernel(const Vec2Args a) {
+    static_assert((SK & (SK - 1)) == 0, "SK is a power of two");
+    __shared__ f32x4 red[(SK > 1 ? SK / 2 : 1) * RT * MT * 64];
+    const int lane = threadIdx.x & 63;
+    const int ks = threadIdx.x >> 6;
+    const int g = lane >> 4, m = lane & 15;
+    const int n0 = blockIdx.x * (RT * 16);
+    const int KB = a.KB;
+    const int per = ((KB + SK - 1) / SK + U - 1) / U * U;  // whole U-groups per wavefront
+    const int kb0 = ks * per, kb1 = min(KB, kb0 + per);
+    const int8_t *wrow[RT];
+    const uint8_t *srow[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int row = min(n0 + rt * 16 + m, a.N - 1);
+        wrow[rt] = FMT == GPHQ_FMT_Q4 ? (const int8_t *)a.codes + (size_t)row * (a.K >> 1) + (g & 1) * 8
+                                      : (const int8_t *)a.codes + (size_t)row * a.K + g * 8;
+        srow[rt] = (const uint8_t *)a.scales + (size_t)row * KB * (FMT == GPHQ_FMT_Q8B_F32 ? 4 : 2);
+    }
+    // The lane's C rows 4g..4g+3 of tile t are vectors t*8 + 2g (hi, lo) and t*8 + 2g + 1.
+    const float *invp[MT][2];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) invp[t][p] = a.inv + (size_t)min(t * 8 + 2 * g + p, a.V - 1) * KB;
+    f32x4 acc[RT][MT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int kbs = kb0; kbs < kb1; kbs += U) {
+        f16x8 av[U][MT];
+        u32x2 w[U][RT];
+        float d[U][RT], iv[U][MT][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kb = min(kbs + u, KB - 1);
+            const bool ok = kbs + u < kb1;
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                av[u][t] = *(const f16x8 *)(a.A + vec_a_offset(t, kb, KB, lane));
+                iv[u][t][0] = ok ? invp[t][0][kb] : 0.0f;
+                iv[u][t][1] = ok ? invp[t][1][kb] : 0.0f;
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                w[u][rt] = *(const u32x2 *)(wrow[rt] + (size_t)kb * (FMT == GPHQ_FMT_Q4 ? 16 : 32));
+                if constexpr (FMT == GPHQ_FMT_Q8B || FMT == GPHQ_FMT_Q4)
+                    d[u][rt] = half_bits_to_float(((const uint16_t *)srow[rt])[kb]);
+                else if constexpr (FMT == GPHQ_FMT_Q8B_F32)
+                    d[u][rt] = ((const float *)srow[rt])[kb];
+                else
+                    d[u][rt] = 1.0f;
+            }
+        }
+        f32x4 c[U][RT][MT];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const f16x8 b = FMT == GPHQ_FMT_Q4 ? u4x8_to_f16(w[u][rt], (g >> 1) * 4) : i8x8_to_f16(w[u][rt]);
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    c[u][rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[u][t], b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const float d0 = d[u][rt] * iv[u][t][0], d1 = d[u][rt] * iv[u][t][1];
+                    acc[rt][t][0] = fmaf(d0, c[u][rt][t][0], acc[rt][t][0]);
+                    acc[rt][t][1] = fmaf(d0, c[u][rt][t][1], acc[rt][t][1]);
+                    acc[rt][t][2] = fmaf(d1, c[u][rt][t][2], acc[rt][t][2]);
+                    acc[rt][t][3] = fmaf(d1, c[u][rt][t][3], acc[rt][t][3]);
+                }
+    }
+#pragma unroll
+    for (int half = SK / 2; half >= 1; half >>= 1) {
+        if (ks >= half && ks < 2 * half) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) red[(((ks - half) * RT + rt) * MT + t) * 64 + lane] = acc[rt][t];
+        }
+        __syncthreads();
+        if (ks < half) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) acc[rt][t] += red[((ks * RT + rt) * MT + t) * 64 + lane];
+        }
+        __syncthreads();
+    }
+    if (ks != 0) return;
+    float nf[MT][2];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) nf[t][p] = 1.0f;
+    if constexpr (NORM) {
+        // Each vector's block sums of squares, added by the whole wavefront in
+        // a fixed order; lane group g keeps vectors t*8 + 2g + {0, 1}.
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int vv = 0; vv < 8; ++vv) {
+                const float *q = a.ssq + (size_t)min(t * 8 + vv, a.V - 1) * KB;
+                float part = 0.0f;
+                for (int kb = lane; kb < KB; kb += 64) part += q[kb];
+                const float tot = wave_sum(part);
+                if ((vv >> 1) == g) nf[t][vv & 1] = 1.0f / sqrtf(tot / (float)a.K + a.eps);
+            }
+        }
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int col = n0 + rt * 16 + m;
+        float rs = 1.0f;
+        if constexpr (FMT == GPHQ_FMT_Q8) rs = ((const float *)a.scales)[min(col, a.N - 1)];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const int v = t * 8 + 2 * g + p;
+                float val = (acc[rt][t][2 * p] + acc[rt][t][2 * p + 1]) * nf[t][p];
+                if constexpr (FMT == GPHQ_FMT_Q8) val *= rs;
+                if constexpr (EPI == VEC_SWIGLU) {
+                    const float up = __shfl_xor(val, 1);  // lane l^1 holds column col^1
+                    if (v < a.V && col < a.N && (col & 1) == 0)
+                        a.y[(size_t)v * a.ystride + (col >> 1)] = val / (1.0f + expf(-val)) * up;
+                } else if (v < a.V && col < a.N) {
+                    if constexpr (EPI == VEC_ADD)
+                        a.y[(size_t)v * a.ystride + col] += val;
+                    else
+                        a.y[(size_t)v * a.ystride + col] = val;
+                }
+            }
+        }
+    }
+}
+
 // How a vecs_kernel launch cuts K: `parts` passes over the block's row tiles,
-// each over SK wavefronts' slices of nb 32-value blocks.
+// each over SK wavefronts' slices of NB 32-value blocks.
 struct VecsShape {
-    int iters, SK, nb, parts;
+    int iters, SK, parts;
     int svec;  // block scales load as one aligned vector per lane
 };
 
-// NB: 32-value blocks per slice, at most (their A fragments stay in registers).
+// NB: 32-value blocks per slice (their A fragments stay in registers).
 template <int FMT, int T, bool PAIR, int NB>
 struct VecsTraits {
     static constexpr bool Q4 = FMT == GPHQ_FMT_Q4;
@@ -194,7 +345,7 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
     const int lane = threadIdx.x & 63;
     const int ks = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int g = lane >> 4, m = lane & 15;
-    const int KB = a.KB, SK = sh.SK, nb = sh.nb, iters = sh.iters, CH = X::ch(SK);
+    const int KB = a.KB, SK = sh.SK, iters = sh.iters, CH = X::ch(SK);
     u32x4 *const st = (u32x4 *)(smem + ks * X::kWave);
     uint8_t *const ssc = smem + ks * X::kWave + X::kStage;
     float *const siv = (float *)(ssc + X::kScale);
@@ -276,10 +427,19 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
         }
     };
     for (int part_i = 0; part_i < sh.parts; ++part_i) {
-        kb0 = min((part_i * SK + ks) * nb, KB);
-        const int mine = min(nb, KB - kb0);  // blocks of this slice (0: none left)
+        kb0 = min((part_i * SK + ks) * NB, KB);
+        const int mine = min(NB, KB - kb0);  // blocks of this slice (0: none left)
         int tt = blockIdx.x;
         gload(tt);
+        // All of the slice's activation loads are issued before the first is used.
+        constexpr int IV = NB * VC / 64;  // block factors per lane
+        static_assert(IV * 64 == NB * VC, "whole wavefronts of block factors");
+        float iv[IV];
+#pragma unroll
+        for (int i = 0; i < IV; ++i) {
+            const int b = (lane + 64 * i) / VC, v = (lane + 64 * i) % VC;
+            iv[i] = a.inv[(size_t)min(v, a.V - 1) * KB + min(kb0 + b, KB - 1)];
+        }
         f16x8 av[NB][AT];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -288,11 +448,8 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
                 if (b < mine) av[b][t] = *(const f16x8 *)(a.A + vec_a_offset(t, kb0 + b, KB, lane));
                 else av[b][t] = f16x8{};
             }
-        for (int e = lane; e < NB * VC; e += 64) {
-            const int b = e / VC, v = e - b * VC;
-            const float iv = a.inv[(size_t)min(v, a.V - 1) * KB + min(kb0 + b, KB - 1)];
-            siv[e] = b < mine ? iv : 0.0f;
-        }
+#pragma unroll
+        for (int i = 0; i < IV; ++i) siv[lane + 64 * i] = (lane + 64 * i) / VC < mine ? iv[i] : 0.0f;
         lwrite();
         for (int it = 0; it < iters; ++it, tt += gridDim.x) {
             const bool more = it + 1 < iters;
@@ -719,23 +876,11 @@ size_t gemv_vec_split_bytes(int V, int K, int N) {
     return parts ? (size_t)parts * V * N * 4 : 0;
 }
 
-static int vech_cus() {
-    static int cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (!cached[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cached[dev] = n;
-    }
-    return cached[dev];
-}
-
 template <int FMT, int SK, int EPI, bool NORM>
 static int go_vech(const Vec2Args &a, hipStream_t stream) {
     const int tiles = (a.N + 15) / 16;
     const int perCu = std::max(1, 8 / SK);  // about 8 wavefronts per CU
-    const int blocks = std::max(1, std::min(tiles, vech_cus() * perCu));
+    const int blocks = std::max(1, std::min(tiles, device_cus() * perCu));
     const int iters = (tiles + blocks - 1) / blocks;
     hipLaunchKernelGGL((vech_kernel<FMT, SK, EPI, NORM, false>), dim3((unsigned)blocks), dim3(64 * SK), 0, stream, a,
                        iters);
@@ -748,7 +893,7 @@ template <int FMT, int EPI, bool NORM>
 static int go_vech_split(const Vec2Args &a, int parts, hipStream_t stream, bool finish) {
     constexpr int SK = kVechMaxSlices;
     const int tiles = (a.N + 15) / 16;
-    const int blocks = std::max(1, std::min(tiles, vech_cus() / parts));
+    const int blocks = std::max(1, std::min(tiles, device_cus() / parts));
     const int iters = (tiles + blocks - 1) / blocks;
     hipLaunchKernelGGL((vech_kernel<FMT, SK, VEC_STORE, false, true>), dim3((unsigned)blocks, (unsigned)parts),
                        dim3(64 * SK), 0, stream, a, iters);
@@ -801,23 +946,18 @@ size_t gemv_vec_workspace_bytes(int V, int K) {
     return (size_t)MT * KB * 1024 + 2 * (size_t)V * KB * 4 + 256;
 }
 
-// The slices of K: as few passes as hold KB blocks, each over as many
-// wavefronts as it has 128-byte lines. Every block reads all of its A
-// fragments, so few blocks of many slices move less than many blocks of few:
-// V = 12, K = 672, N = 9000, Q8B takes 12 us at two blocks of five slices a CU,
-// 10 us at one. Where the tiles' sums of a further pass would not fit in LDS,
-// more blocks walk fewer tiles.
+// The slices of K: as few passes as hold KB blocks, each over as few wavefronts
+// as hold a pass's share (twice the wavefronts at half the blocks each took
+// 8 vectors, K = 1376, N = 24000, Q8B 17.7 us, 14.4 with this). Where the tiles'
+// sums of a further pass would not fit in LDS, more blocks walk fewer tiles.
 template <int FMT, int T, bool PAIR, int NB, int EPI, bool NORM>
 static int go_vecs(const Vec2Args &a, hipStream_t stream) {
     using X = VecsTraits<FMT, T, PAIR, NB>;
     constexpr int kMaxSK = X::kMaxSK, kLds = 160 << 10;
-    const int line = X::Q4 ? 8 : 4;  // blocks per 128-byte line
     VecsShape sh{};
     sh.parts = (a.KB + kMaxSK * NB - 1) / (kMaxSK * NB);
     const int per = (a.KB + sh.parts - 1) / sh.parts;  // blocks of one pass
-    sh.SK = std::min(kMaxSK, (per + line - 1) / line);
-    sh.nb = std::min(NB, ((per + sh.SK - 1) / sh.SK + line - 1) / line * line);
-    sh.SK = (per + sh.nb - 1) / sh.nb;
+    sh.SK = (per + NB - 1) / NB;
     sh.svec = X::SB && a.KB % 4 == 0 && (uintptr_t)a.scales % 16 == 0;
     const int tiles = (a.N + 15) / 16;
     int blocks = std::max(1, std::min(tiles, device_cus() * std::max(1, (T == 1 && !PAIR ? kMaxSK : 8) / sh.SK)));
@@ -827,8 +967,8 @@ static int go_vecs(const Vec2Args &a, hipStream_t stream) {
     blocks = (tiles + sh.iters - 1) / sh.iters;
     const int lds = X::lds(sh.SK, sh.parts, sh.iters);
     if (lds > (64 << 10))
-        (void)hipFuncSetAttribute((const void *)vecs_kernel<FMT, T, PAIR, NB, EPI, NORM>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        GPHQ_TRY(hip_status(hipFuncSetAttribute((const void *)vecs_kernel<FMT, T, PAIR, NB, EPI, NORM>,
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds)));
     hipLaunchKernelGGL((vecs_kernel<FMT, T, PAIR, NB, EPI, NORM>), dim3((unsigned)blocks), dim3(64 * sh.SK), lds, stream,
                        a, sh);
     return launch_status();
@@ -851,13 +991,70 @@ static int launch_vecs_tiles(const Vec2Args &a, hipStream_t stream) {
     return GPHQ_ERR_UNSUPPORTED;
 }
 
+// Weight rows per block of vecd_kernel for this product (16 or 64), or 0 when
+// vecs_kernel takes it. vecd_kernel is the faster where vecs_kernel's slices are
+// few or fill only in part, so that its LDS round trip and barriers are most of
+// its time, and where few blocks read the A fragments (each block of 16 rows
+// reads all of them). Per vectors (<= 8, <= 16, more) and format: at most onePass
+// blocks of K where vecs_kernel needs one pass, or perPass in each of two or
+// three, at most `work` tiles x blocks and at most maxTiles tiles of 16 rows. Fitted on MI355X to K = 32 to 4128 and N =
+// 64 to 24000, vecd / vecs in us: 16 vectors, Q8B, 480 -> 3000 5.7 / 7.0, 928 ->
+// 5000 8.7 / 8.6, 1632 -> 5000 11.5 / 10.6, 480 -> 24000 11.0 / 10.7; 1 vector,
+// Q8, 928 -> 5000 6.4 / 6.9, 2080 -> 6144 10.6 / 9.8; 8 vectors, Q4, 480 -> 3000
+// 5.1 / 5.8, 928 -> 6144 7.3 / 6.8; 32 vectors, Q8B, 928 -> 4096 8.8 / 10.0,
+// 3168 -> 5000 35.8 / 25.5; 17 vectors, Q4, one whole pass, 2048 -> 6144 16.7 /
+// 12.2, one block more, 2080 -> 5000 15.0 / 16.4. 64-row blocks of eight slices:
+// 17-24 vectors just past one pass (Q4, 2080 -> 16000: 21.8 / 26.1), as long as
+// they are one round of the chip (24000: 36.5 / 35.6; Q8B_F32, 2336 -> 16000: 28.6 / 24.8).
+static int vecd_rows(int fmt, int V, int KB, int N) {
+    static constexpr struct {
+        int onePass, perPass, work, maxTiles;
+    } kRules[3][3] = {{{52, 0, 20000, INT32_MAX}, {26, 0, 10000, INT32_MAX}, {18, 0, 6000, INT32_MAX}},
+                      {{30, 0, 18000, 1024}, {36, 0, 18000, 1024}, {16, 0, 6000, 1024}},
+                      {{52, 52, 22000, 600}, {44, 44, 18000, 600}, {30, 37, 26000, 400}}};
+    const auto &r = kRules[V <= 8 ? 0 : V <= 16 ? 1 : 2][fmt == GPHQ_FMT_Q8 ? 0 : fmt == GPHQ_FMT_Q4 ? 2 : 1];
+    const long tiles = ((long)N + 15) / 16;
+    const int pass = V > 16 ? 64 : 128, parts = (KB + pass - 1) / pass;
+    if (V > 16 && V <= 24 && fmt != GPHQ_FMT_Q8B_F32 && KB > pass && KB <= 80 && tiles > 2 * device_cus() &&
+        tiles <= 4 * device_cus())
+        return 64;
+    const bool few = parts == 1 ? KB <= r.onePass : parts <= 3 && KB <= r.perPass * parts;
+    return few && KB * tiles <= r.work && tiles <= r.maxTiles ? 16 : 0;
+}
+
+template <int FMT, int MT, int EPI, bool NORM>
+static int go_vecd(const Vec2Args &a, int rows, hipStream_t stream) {
+    if constexpr (MT == 3) {
+        if (rows == 64) {
+            hipLaunchKernelGGL((vecd_kernel<FMT, MT, 8, 4, 2, EPI, NORM>), dim3((unsigned)((a.N + 63) / 64)), dim3(512),
+                               0, stream, a);
+            return launch_status();
+        }
+    }
+    hipLaunchKernelGGL((vecd_kernel<FMT, MT, 4, 1, 4, EPI, NORM>), dim3((unsigned)((a.N + 15) / 16)), dim3(256), 0,
+                       stream, a);
+    return launch_status();
+}
+
+template <int FMT, int EPI, bool NORM>
+static int launch_vecs_fmt(const Vec2Args &a, int rows, hipStream_t stream) {
+    if (!rows) return launch_vecs_tiles<FMT, EPI, NORM>(a, stream);
+    switch ((2 * a.V + 15) / 16) {
+    case 1: return go_vecd<FMT, 1, EPI, NORM>(a, rows, stream);
+    case 2: return go_vecd<FMT, 2, EPI, NORM>(a, rows, stream);
+    case 3: return go_vecd<FMT, 3, EPI, NORM>(a, rows, stream);
+    case 4: return go_vecd<FMT, 4, EPI, NORM>(a, rows, stream);
+    }
+    return GPHQ_ERR_UNSUPPORTED;
+}
+
 template <int EPI, bool NORM>
-static int launch_vecs(int fmt, const Vec2Args &a, hipStream_t stream) {
+static int launch_vecs(int fmt, const Vec2Args &a, int rows, hipStream_t stream) {
     switch (fmt) {
-    case GPHQ_FMT_Q8: return launch_vecs_tiles<GPHQ_FMT_Q8, EPI, NORM>(a, stream);
-    case GPHQ_FMT_Q8B: return launch_vecs_tiles<GPHQ_FMT_Q8B, EPI, NORM>(a, stream);
-    case GPHQ_FMT_Q8B_F32: return launch_vecs_tiles<GPHQ_FMT_Q8B_F32, EPI, NORM>(a, stream);
-    case GPHQ_FMT_Q4: return launch_vecs_tiles<GPHQ_FMT_Q4, EPI, NORM>(a, stream);
+    case GPHQ_FMT_Q8: return launch_vecs_fmt<GPHQ_FMT_Q8, EPI, NORM>(a, rows, stream);
+    case GPHQ_FMT_Q8B: return launch_vecs_fmt<GPHQ_FMT_Q8B, EPI, NORM>(a, rows, stream);
+    case GPHQ_FMT_Q8B_F32: return launch_vecs_fmt<GPHQ_FMT_Q8B_F32, EPI, NORM>(a, rows, stream);
+    case GPHQ_FMT_Q4: return launch_vecs_fmt<GPHQ_FMT_Q4, EPI, NORM>(a, rows, stream);
     }
     return GPHQ_ERR_UNSUPPORTED;
 }
@@ -929,16 +1126,17 @@ int gemv_vec_fused_launch(int fmt, int norm, int epi, const void *codes, const v
         else hipLaunchKernelGGL(vec_empty_kernel<GPHQ_FMT_Q8B>, grid, dim3(256), 0, stream, a, epi == VEC_STORE);
         return launch_status();
     }
+    const int rows = vecd_rows(fmt, V, KB, N);
     // A rows past the vectors are never written; they only feed results that
     // are never stored.
     hipLaunchKernelGGL(vec_prep_blocks_kernel, dim3((unsigned)(((long)V * KB * 4 + 255) / 256)), dim3(256), 0, stream,
-                       x, xstride, V, KB, A, inv, ssq);
+                       x, xstride, V, KB, A, inv, ssq, !rows && vec_pair(V));
     GPHQ_TRY(launch_status());
-    if (epi == VEC_ADD) return norm ? launch_vecs<VEC_ADD, true>(fmt, a, stream)
-                                    : launch_vecs<VEC_ADD, false>(fmt, a, stream);
-    if (epi == VEC_SWIGLU) return norm ? launch_vecs<VEC_SWIGLU, true>(fmt, a, stream)
-                                       : launch_vecs<VEC_SWIGLU, false>(fmt, a, stream);
-    return norm ? launch_vecs<VEC_STORE, true>(fmt, a, stream) : launch_vecs<VEC_STORE, false>(fmt, a, stream);
+    if (epi == VEC_ADD) return norm ? launch_vecs<VEC_ADD, true>(fmt, a, rows, stream)
+                                    : launch_vecs<VEC_ADD, false>(fmt, a, rows, stream);
+    if (epi == VEC_SWIGLU) return norm ? launch_vecs<VEC_SWIGLU, true>(fmt, a, rows, stream)
+                                       : launch_vecs<VEC_SWIGLU, false>(fmt, a, rows, stream);
+    return norm ? launch_vecs<VEC_STORE, true>(fmt, a, rows, stream) : launch_vecs<VEC_STORE, false>(fmt, a, rows, stream);
 }
 
 // y[v*ystride + j] for v < V (gphq_gemv_vec). Arguments were validated by the caller.

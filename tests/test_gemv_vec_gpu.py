@@ -127,6 +127,47 @@ def test_slice_and_pass_edges(fmt, k, n):
             assert finite and rel <= 1e-5, (lanes, v, rel)
 
 
+@pytest.mark.parametrize("fmt,lanes,k,n", [
+    # more tiles a block than one reduction group, in one pass (the whole group and a remainder)
+    (orc.FMT_Q4, 8, 4096, 24581), (orc.FMT_Q8B, 3, 1376, 40011),
+    # several groups in several passes: a hi/lo pair, three and four tiles
+    (orc.FMT_Q8B, 16, 4128, 20000), (orc.FMT_Q8B_F32, 24, 4128, 12300), (orc.FMT_Q8, 32, 4128, 12300),
+    # more tiles a block than its LDS holds between passes
+    (orc.FMT_Q4, 32, 3648, 75000),
+    # 64-row blocks, the last one cut
+    (orc.FMT_Q8, 17, 2080, 16000), (orc.FMT_Q8B, 24, 2336, 9001),
+    # few rows past the small products' sizes: partial last slices and passes
+    (orc.FMT_Q8, 5, 1700, 17), (orc.FMT_Q8, 17, 4256, 1), (orc.FMT_Q8B, 9, 1248, 40), (orc.FMT_Q8B_F32, 32, 2720, 33),
+    (orc.FMT_Q4, 2, 608, 100), (orc.FMT_Q4, 12, 8256, 31),
+])
+def test_persistent_groups_and_passes(fmt, lanes, k, n):
+    """Sampled rows of each lane against float64, with gaps between the vectors and between the outputs."""
+    import torch
+
+    k -= k % 32
+    gen = torch.Generator(device="cuda").manual_seed(k + n + lanes)
+    codes = torch.randint(0, 256, (n, k // 2 if fmt == orc.FMT_Q4 else k), dtype=torch.uint8, device="cuda", generator=gen)
+    scales = torch.rand((n, 1 if fmt == orc.FMT_Q8 else k // 32), device="cuda", generator=gen) * 0.01
+    if fmt in (orc.FMT_Q8B, orc.FMT_Q4):
+        scales = scales.half()
+    xs, ys = k + 4, n + 3
+    x = torch.randn((lanes, xs), device="cuda", generator=gen)
+    y = torch.full((lanes, ys), -7.0, device="cuda")
+    work = torch.empty(gphq.gemv_vec_workspace_bytes(lanes, k), dtype=torch.uint8, device="cuda")
+    gphq.gemv_vec(fmt, codes, scales, x, y, lanes, k, n, work, x_stride=xs, y_stride=ys)
+    rng = np.random.default_rng(n)
+    rows = np.unique(np.concatenate([np.arange(min(n, 16)), np.arange(max(0, n - 40), n), rng.integers(0, n, 400)]))
+    at = torch.from_numpy(rows).cuda()
+    c, s, got = host(codes[at]), host(scales[at]), host(y)
+    c = c.ravel() if fmt == orc.FMT_Q4 else c.ravel().view(np.int8)
+    s = s.ravel().view(np.uint16) if fmt in (orc.FMT_Q8B, orc.FMT_Q4) else s.ravel()
+    assert (got[:, n:] == -7.0).all()
+    for v in range(lanes):
+        want = orc.gemv_f64(fmt, c, s, host(x[v, :k]), k, len(rows))[0]
+        _, rel, finite = vector_error(want, got[v, rows])
+        assert finite and rel <= 1e-5, (v, rel)
+
+
 def test_strides_leave_gaps_untouched():
     k, n, lanes, xs, ys = 512, 48, 5, 600, 64
     rng = np.random.default_rng(3)
