@@ -7,10 +7,12 @@
 // with dot_b the exact int32 block product, so results are bit-exact against
 // the oracle's restatement of that sum.
 //
-// v_mfma_i32_32x32x32_i8 takes exactly one 32-value block per instruction, so
-// every block's int32 products come out of one MFMA with a zero accumulator;
-// the fp32 scale-accumulate that follows is VALU work (three instructions per
-// output and block), which bounds this kernel well below the int8 MFMA rate.
+// One v_mfma_i32_16x16x32_i8 (q8b_tile_kernel, up to 16 rows q8b_small_kernel)
+// or v_mfma_i32_32x32x32_i8 (q8b_gemm_kernel, the 128 x 192 tiles) takes exactly
+// one 32-value block, so every block's int32 products come out of one MFMA with
+// a zero accumulator; the fp32 scale-accumulate that follows is VALU work (three
+// instructions per output and block), which bounds these kernels well below the
+// int8 MFMA rate. One row takes sdot4 chains (q8b_gemv_kernel).
 #include <type_traits>
 
 #include "common.h"
@@ -464,27 +466,26 @@ __global__ __launch_bounds__(64 * WGM * WGN) void q8b_tile_kernel(const Q8bArgs 
         }
 }
 
-// M <= 16 * TI: one wavefront (and block) per 16 weight rows, all
-// activation rows in TI tiles of 16. A step is 128 bytes of K (four
-// blocks): the wavefront loads its 16 weight rows and 16 * TI activation
+// M <= 16: one wavefront (and block) per 16 weight rows, all activation rows
+// in one tile. A step is 128 bytes of K (four
+// blocks): the wavefront loads its 16 weight rows and 16 activation
 // rows with 16-byte loads, eight lanes per row (whole 128-byte lines), their
 // block scales with one float per lane, and keeps D steps of loads in
 // flight in a register ring. Each step passes through the wavefront's own
 // LDS (rows padded to 144 bytes), from which every block is one
-// v_mfma_i32_16x16x32_i8 per activation tile (lane l supplies bytes
+// v_mfma_i32_16x16x32_i8 (lane l supplies bytes
 // 8(l/16)..+8 of the block for row or column l%16 and receives rows
 // 4(l/16)..+3 of column l%16). The chain per output is the tiled kernel's,
 // in block order: acc = fmaf(float(dot_b), da * dw, acc), so the results
 // are the same bit for bit.
-template <int TI, int D>
+template <int D>
 __global__ __launch_bounds__(64) void q8b_small_kernel(const Q8bArgs a) {
     constexpr int RS = 144;             // LDS row stride of the code tiles, bytes
-    constexpr int AR = 16 * TI;         // activation rows
     static_assert(D % 2 == 0, "the ring pairs with two LDS buffers");
     __shared__ __align__(16) int8_t wl[2][16 * RS];
-    __shared__ __align__(16) int8_t al[2][AR * RS];
+    __shared__ __align__(16) int8_t al[2][16 * RS];
     __shared__ float swl[2][16][4];                // [buffer][weight row][block of the step]
-    __shared__ __align__(16) float sal[2][4][AR];  // [buffer][block of the step][activation row]
+    __shared__ __align__(16) float sal[2][4][16];  // [buffer][block of the step][activation row]
     const int lane = threadIdx.x, kb = a.k >> 5, steps = kb >> 2;
     const int n0 = blockIdx.x * 16;
     const int lr = lane >> 3, lc = lane & 7;  // loader: row lr (+8h), 16-byte chunk lc
@@ -492,17 +493,14 @@ __global__ __launch_bounds__(64) void q8b_small_kernel(const Q8bArgs a) {
     const int8_t *wp[2];
     wp[0] = a.qw + (size_t)min(n0 + lr, a.n - 1) * a.k + lc * 16;
     wp[1] = a.qw + (size_t)min(n0 + lr + 8, a.n - 1) * a.k + lc * 16;
-    const int8_t *ap[2 * TI];
+    const int8_t *ap[2];
 #pragma unroll
-    for (int h = 0; h < 2 * TI; ++h) ap[h] = a.qa + (size_t)min(lr + 8 * h, a.m - 1) * a.k + lc * 16;
-    // Scales: lane l takes block l%4 of the step of weight row l/4 and of
-    // activation rows l/4 + 16i.
+    for (int h = 0; h < 2; ++h) ap[h] = a.qa + (size_t)min(lr + 8 * h, a.m - 1) * a.k + lc * 16;
+    // Scales: lane l takes block l%4 of the step of weight and activation row l/4.
     const float *dwp = a.dw + (size_t)min(n0 + (lane >> 2), a.n - 1) * kb + (lane & 3);
-    const float *dap[TI];
-#pragma unroll
-    for (int i = 0; i < TI; ++i) dap[i] = a.da + (size_t)min((lane >> 2) + 16 * i, a.m - 1) * kb + (lane & 3);
-    i32x4 wr[D][2], ar[D][2 * TI];
-    float sw[D], sa[D][TI];
+    const float *dap = a.da + (size_t)min(lane >> 2, a.m - 1) * kb + (lane & 3);
+    i32x4 wr[D][2], ar[D][2];
+    float sw[D], sa[D];
     auto load = [&](int p, int st, bool first) {
         const size_t off = (size_t)st * 128;
         auto ld = [&](const int8_t *q, bool stream) -> i32x4 {
@@ -521,24 +519,20 @@ __global__ __launch_bounds__(64) void q8b_small_kernel(const Q8bArgs a) {
         wr[p][0] = ld(wp[0] + off, true);
         wr[p][1] = ld(wp[1] + off, true);
 #pragma unroll
-        for (int h = 0; h < 2 * TI; ++h) ar[p][h] = ld(ap[h] + off, false);
+        for (int h = 0; h < 2; ++h) ar[p][h] = ld(ap[h] + off, false);
         sw[p] = lf(dwp + 4 * st);
-#pragma unroll
-        for (int i = 0; i < TI; ++i) sa[p][i] = lf(dap[i] + 4 * st);
+        sa[p] = lf(dap + 4 * st);
     };
     // Ring slot p to LDS buffer buf (this wavefront alone reads it back).
     auto stage = [&](int p, int buf) {
         *(i32x4 *)&wl[buf][lr * RS + lc * 16] = wr[p][0];
         *(i32x4 *)&wl[buf][(lr + 8) * RS + lc * 16] = wr[p][1];
 #pragma unroll
-        for (int h = 0; h < 2 * TI; ++h) *(i32x4 *)&al[buf][(lr + 8 * h) * RS + lc * 16] = ar[p][h];
+        for (int h = 0; h < 2; ++h) *(i32x4 *)&al[buf][(lr + 8 * h) * RS + lc * 16] = ar[p][h];
         swl[buf][lane >> 2][lane & 3] = sw[p];
-#pragma unroll
-        for (int i = 0; i < TI; ++i) sal[buf][lane & 3][(lane >> 2) + 16 * i] = sa[p][i];
+        sal[buf][lane & 3][lane >> 2] = sa[p];
     };
-    f32x4 acc[TI];
-#pragma unroll
-    for (int i = 0; i < TI; ++i) acc[i] = f32x4{};
+    f32x4 acc = f32x4{};
 #pragma unroll
     for (int p = 0; p < D; ++p) load(p, min(p, steps - 1), true);
     stage(0, 0);
@@ -558,15 +552,12 @@ __global__ __launch_bounds__(64) void q8b_small_kernel(const Q8bArgs a) {
             for (int b = 0; b < 4; ++b) {
                 const long wv = *(const long *)&wl[cur][c * RS + 32 * b + 8 * g];
                 const float w1 = swl[cur][c][b];
+                const long av = *(const long *)&al[cur][c * RS + 32 * b + 8 * g];
+                const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, wv, i32x4{}, 0, 0, 0);
+                const float4 s4 = *(const float4 *)&sal[cur][b][4 * g];
+                const float s_[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
-                for (int i = 0; i < TI; ++i) {
-                    const long av = *(const long *)&al[cur][(16 * i + c) * RS + 32 * b + 8 * g];
-                    const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, wv, i32x4{}, 0, 0, 0);
-                    const float4 s4 = *(const float4 *)&sal[cur][b][16 * i + 4 * g];
-                    const float s_[4] = {s4.x, s4.y, s4.z, s4.w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf((float)d[e], __fmul_rn(s_[e], w1), acc[i][e]);
-                }
+                for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf((float)d[e], __fmul_rn(s_[e], w1), acc[e]);
             }
             __builtin_amdgcn_wave_barrier();
             if (st + 1 >= steps) break;
@@ -575,12 +566,10 @@ __global__ __launch_bounds__(64) void q8b_small_kernel(const Q8bArgs a) {
     const int col = n0 + c;
     if (col < a.n) {
 #pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = 16 * i + 4 * g + e;
-                if (row < a.m) a.y[(size_t)row * a.n + col] = acc[i][e];
-            }
+        for (int e = 0; e < 4; ++e) {
+            const int row = 4 * g + e;
+            if (row < a.m) a.y[(size_t)row * a.n + col] = acc[e];
+        }
     }
 }
 
@@ -674,9 +663,9 @@ int go_gemv(const Q8bArgs &a, hipStream_t st) {
     return launch_status();
 }
 
-template <int TI, int D>
+template <int D>
 int go_small(const Q8bArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL((q8b_small_kernel<TI, D>), dim3((unsigned)((a.n + 15) / 16)), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((q8b_small_kernel<D>), dim3((unsigned)((a.n + 15) / 16)), dim3(64), 0, st, a);
     return launch_status();
 }
 
@@ -791,7 +780,7 @@ int gphq_q8b_gemm(const int8_t *qa_dev, const float *da_dev, const int8_t *qw_de
         case 12288: return go_gemv<12>(a, st);
         }
     }
-    return go_small<1, 8>(a, st);  // a ring of eight steps in flight
+    return go_small<8>(a, st);  // a ring of eight steps in flight
 }
 
 }  // extern "C"
