@@ -17,8 +17,8 @@ with MulPanelsI8's scaling (float32(sum) * weight scale) * row scale
   code boundary may take the neighbouring code. One flipped code k moves an
   output row by (max|x| / 127) * |W[:, k]|, relative (max/rms) / (127 sqrt(K))
   of the row: about 9e-4 at K = 1024, doubled by SwiGLU's product. Rows are
-  held to relative L2 5e-3 (a flip or two) and 95% of them to 1e-5 (no
-  flip: a wrong scale, order or gate/up pairing fails every row).
+  held to relative L2 5e-3 (a flip or two) and 95% of them (at K = 4096, with
+  four times the values that can flip, 84%) to 1e-5 (no flip: a wrong scale, order or gate/up pairing fails every row).
 * Whole passes: past the first projection, inputs differ from the oracle's
   by the FP16 attention's rounding (about 1e-3 relative), and quantizing
   them turns that into code flips in a few percent of the values, as large
@@ -131,10 +131,11 @@ def test_project_int8_tile_shapes_bit_exact(rows):
     test_project_int8_residual_add_bit_exact(lc.SMALL_06B, 3, rows)
 
 
-@pytest.mark.parametrize("rows", [40, 400, 1500, 3000])
+@pytest.mark.parametrize("rows", [40, 400, 1500, 3000, 4500])
 def test_project_int8_odd_steps_bit_exact(rows):
     """K = 1088 = 17 steps of 64: the whole-line loads' last piece is half a line
-    (3000 rows: 256 x 256 tiles). Sums from a float64 product of the codes."""
+    (3000 rows: 256 x 256 tiles; 4500 rows: 256 x 128 ones past the last whole
+    round). Sums from a float64 product of the codes."""
     import torch
 
     geom = lo.Geometry(hidden=4096, layers=1, heads=32, kv_heads=8, head_dim=128, inter=1088, vocab=256, max_pos=64)
@@ -157,12 +158,10 @@ def test_project_int8_odd_steps_bit_exact(rows):
     assert np.array_equal(got.view(np.uint32), (y0 + v).astype(np.float32).view(np.uint32))
 
 
-@pytest.mark.parametrize("proj", [0, 2])
-@pytest.mark.parametrize("rows", [1, 64, 257])
-def test_project_int8_normalized_inputs(proj, rows):
+def _check_normalized(geom, proj, rows):
     import torch
 
-    model, oracle, lm = setup(lc.SMALL_06B, lo.FMT_Q8, seed=6)
+    model, _, lm = setup(geom, lo.FMT_Q8, seed=6)
     W, sw, n, k = _layer_weights(model, proj)
     g = model["geom"]
     rng = np.random.default_rng(7 * proj + rows)
@@ -184,7 +183,24 @@ def test_project_int8_normalized_inputs(proj, rows):
     err = rel_rows(y, got)
     print(f"  max row rel {err.max():.3g}, median {np.median(err):.3g}")
     assert err.max() <= 5e-3, err.max()
-    assert np.mean(err <= 1e-5) >= 0.95, np.sort(err)[-10:]
+    # A value within fp32 rounding of a tie (about 1.2e-5 of them: 127 levels, typical |q| 35, 2^-23) may take the
+    # other code, and one is enough to move its row: at most about three times that share of the rows.
+    assert np.mean(err <= 1e-5) >= min(0.95, 1.0 - 4e-5 * k), np.sort(err)[-10:]
+
+
+@pytest.mark.parametrize("proj", [0, 2])
+@pytest.mark.parametrize("rows", [1, 64, 257])
+def test_project_int8_normalized_inputs(proj, rows):
+    _check_normalized(lc.SMALL_06B, proj, rows)
+
+
+@pytest.mark.parametrize("hidden,proj,rows", [(1024, 0, 1030), (1024, 0, 2500), (4096, 0, 3000), (1024, 2, 700),
+                                              (1024, 2, 1500), (1024, 2, 3000)])
+def test_project_int8_wide_tiles(hidden, proj, rows):
+    """Every row of the whole-line kernel's store and SwiGLU epilogues: 256 x 128 and 256 x 256 tiles, and 256 x 256
+    ones followed by 256 x 128 from a later column (at 256 CUs, in this order)."""
+    wide = lo.Geometry(hidden=4096, layers=1, heads=32, kv_heads=8, head_dim=128, inter=1088, vocab=256, max_pos=64)
+    _check_normalized(wide if hidden == 4096 else lc.SMALL_06B, proj, rows)
 
 
 @pytest.mark.parametrize("rows", [64, 16, 1], ids=["one_pass", "passes_of_16", "one_token_passes"])

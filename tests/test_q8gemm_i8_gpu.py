@@ -71,12 +71,10 @@ def oracle_out(x, rows, k, q, scales, n):
 SHAPES = [(1, 4, 1), (3, 7, 17), (12, 64, 64), (16, 257, 129), (12, 4096, 1024), (5, 12288, 64), (1, 32, 64),
           (1, 4096, 1024), (1, 12288, 200), (1, 96, 5), (17, 100, 33), (64, 640, 96), (100, 512, 300),
           (200, 1024, 520),
-          # 17..256 rows, K a multiple of 256: one-stage K,
-          # column tiles past N in a block, two row blocks
+          # few columns (64 x 16 tiles): K a multiple of 256 and not, one to
+          # three row blocks, columns past the last whole tile
           (24, 256, 200), (48, 256, 500), (130, 1024, 64), (256, 2048, 77), (33, 12288, 48),
-          # 129..512 rows, K not a multiple of 256
           (300, 640, 260), (512, 192, 200), (140, 64, 40),
-          # K not a multiple of 256 from 65 rows and past 512 rows
           (100, 640, 200), (600, 320, 130)]
 
 
@@ -125,12 +123,14 @@ def test_config2_shapes_bit_exact(m):
 
 @pytest.mark.parametrize("m,n", [(17, 50), (31, 12200), (50, 4500), (64, 9000), (100, 5000), (110, 7800), (129, 3000),
                                  (130, 9300), (190, 12240), (257, 20000), (300, 9000), (520, 12300), (1030, 8200),
-                                 (1100, 16000)])
-@pytest.mark.parametrize("k", [64, 65, 190, 256, 735])
+                                 (1100, 16000), (17, 12295), (70, 8300), (140, 6300), (260, 10890)])
+@pytest.mark.parametrize("k", [64, 65, 190, 256, 735, 1793])
 def test_tile_shapes_and_last_steps_bit_exact(m, n, k):
-    """Every tile shape of the dispatch over 1, 2, 3, 4 and 12 K-steps (fewer
-    than the ring's stages, and last stages cut short), partial row and column
-    tiles: exact integer sums from a float64 product of the codes."""
+    """Every tile shape of the dispatch (at 256 CUs) over 1, 2, 3, 4, 12 and 29
+    K-steps (fewer and more than the ring holds, last stages cut short), partial
+    row and column tiles: exact integer sums from a float64 product of the
+    codes. The last four sizes are 64 x 64, 128 x 48, 128 x 64 and 128 x 192 at
+    every K."""
     rng = np.random.default_rng(m + n + k)
     q = rng.integers(-127, 128, k * n).astype(np.int8)
     scales = (np.abs(rng.standard_normal(n)) * 0.01).astype(np.float32)
@@ -142,6 +142,34 @@ def test_tile_shapes_and_last_steps_bit_exact(m, n, k):
     acc = host(dev(qa.astype(np.float64)) @ dev(q.reshape(n, k).astype(np.float64)).T)
     want = (acc.astype(np.float32) * scales[None, :]).astype(np.float32) * rs[:, None]
     assert np.array_equal(got.reshape(m, n).view(np.uint32), want.astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("m,n", [(100, 1500), (50, 4500), (31, 12200), (120, 4500), (70, 6300), (20, 12400), (70, 8300),
+                                 (140, 6300), (140, 8400), (140, 12500), (260, 10980), (520, 13200)])
+@pytest.mark.parametrize("k", [190, 1000])
+def test_tile_shapes_on_strip_ranges(m, n, k):
+    """Each tile shape of the dispatch, in its order at 256 CUs, on strips [1, .) and on a panel range, with a padded
+    output stride: whole 128-byte lines pair column tiles from an odd first tile, nothing outside the range is
+    written."""
+    rng = np.random.default_rng(m + n + k)
+    q = rng.integers(-127, 128, k * n).astype(np.int8)
+    scales = (np.abs(rng.standard_normal(n)) * 0.01).astype(np.float32)
+    w = gphq.WeightsI8(k, n)
+    w.pack(q, scales)
+    x = rng.standard_normal(m * k).astype(np.float32)
+    ws = gphq.WorkspaceI8(k, m)
+    ws.pack(dev(x), m, k)
+    qa, rs, _ = orc.i8_pack_rows(x, m, k)
+    acc = host(dev(qa.astype(np.float64)) @ dev(q.reshape(n, k).astype(np.float64)).T)
+    want = (acc.astype(np.float32) * scales[None, :]).astype(np.float32) * rs[:, None]
+    for mul, width, r0, r1, stride in ((gphq.mul_strips_i8, 16, 1, w.strips() - 1, n + 5),
+                                       (gphq.mul_panels_i8, 64, 1, w.panels(), n + 32)):
+        dst = fill(m * stride)
+        mul(dst, stride, ws, w, r0, r1)
+        got = host(dst).reshape(m, stride)
+        c0, c1 = r0 * width, min(n, r1 * width)
+        assert np.all(got[:, :c0] == -7) and np.all(got[:, c1:] == -7)
+        assert np.array_equal(got[:, c0:c1].view(np.uint32), want[:, c0:c1].astype(np.float32).view(np.uint32))
 
 
 def test_golden_tile():
