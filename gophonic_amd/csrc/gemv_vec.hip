@@ -474,9 +474,10 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
                     else if constexpr (SB == 4) d = __builtin_bit_cast(float, sw[b]);
 #pragma unroll
                     for (int t = 0; t < T; ++t) {
-                        f32x4 cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[b][t], bf, f32x4{0.f, 0.f, 0.f, 0.f}, 0,
-                                                                          0, 0);
-                        if constexpr (PAIR) cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[b][1], bf, cc, 0, 0, 0);
+                        const f32x4 zero{0.f, 0.f, 0.f, 0.f};
+                        f32x4 cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[b][t], bf, zero, 0, 0, 0);
+                        // Added outside: an MFMA with a sum to start from rounds worse.
+                        if constexpr (PAIR) cc += __builtin_amdgcn_mfma_f32_16x16x32_f16(av[b][1], bf, zero, 0, 0, 0);
                         const float *iv = siv + b * VC + (PAIR ? 4 * g : 8 * t + 2 * g);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
@@ -533,13 +534,23 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
             if (slot != CH - 1 && it != iters - 1) continue;  // the same for every wavefront
             __syncthreads();
             if (ks <= slot) {
-                // Wavefront ks adds slot ks's slices in order: the tile slot - ks blocks back.
+                // Wavefront ks adds slot ks's slices (T == 1: the even and the
+                // odd ones apart): the tile slot - ks blocks back.
                 f32x4 r[T];
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
                     const f32x4 *ps = part + (ks * SK * T + t) * 64 + lane;
                     r[t] = ps[0];
-                    for (int k2 = 1; k2 < SK; ++k2) r[t] += ps[k2 * T * 64];
+                    if constexpr (T == 1) {
+                        f32x4 odd = ps[64];
+                        for (int k2 = 2; k2 < SK; k2 += 2) {
+                            r[t] += ps[k2 * 64];
+                            if (k2 + 1 < SK) odd += ps[(k2 + 1) * 64];
+                        }
+                        r[t] += odd;
+                    } else {
+                        for (int k2 = 1; k2 < SK; ++k2) r[t] += ps[k2 * T * 64];
+                    }
                 }
                 epilogue(it - (slot - ks), tt - (slot - ks) * (int)gridDim.x, r);
             }

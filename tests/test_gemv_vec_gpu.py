@@ -168,6 +168,30 @@ def test_persistent_groups_and_passes(fmt, lanes, k, n):
         assert finite and rel <= 1e-5, (v, rel)
 
 
+def test_pair_layout_keeps_the_rounding():
+    """9 to 16 vectors (hi and lo tiles) against the same vectors among 24 (hi and lo rows): the same sums over other
+    slices. Measured on 72000 outputs, 1.06 times the error of the second; 1.18 with lo added inside the hi
+    products' MFMA."""
+    import torch
+
+    k, n = 4096, 6000
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    codes = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    scales = (torch.rand((n, k // 32), device="cuda", generator=gen) * 0.01 + 0.005).half()
+    x = torch.randn((24, k), device="cuda", generator=gen)
+    x[:, 5::256] *= 8
+    b = codes.view(n, k // 32, 16)
+    w = ((torch.cat([b & 15, b >> 4], 2).double() - 8) * scales.double().unsqueeze(2)).view(n, k)
+    want = x[:12].double() @ w.T
+    rel = {}
+    for lanes in (12, 24):
+        y = torch.empty((lanes, n), device="cuda")
+        work = torch.empty(gphq.gemv_vec_workspace_bytes(lanes, k), dtype=torch.uint8, device="cuda")
+        gphq.gemv_vec(orc.FMT_Q4, codes, scales, x, y, lanes, k, n, work)
+        rel[lanes] = float((y[:12].double() - want).norm() / want.norm())
+    assert rel[12] <= 1.12 * rel[24], rel
+
+
 def test_strides_leave_gaps_untouched():
     k, n, lanes, xs, ys = 512, 48, 5, 600, 64
     rng = np.random.default_rng(3)
