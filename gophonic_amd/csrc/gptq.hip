@@ -197,19 +197,27 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
 #pragma unroll
     for (int x = 0; x < MT; ++x)
 #pragma unroll
-        for (int y = 0; y < NT; ++y)
+        for (int y = 0; y < NT; ++y) {
+            const int i0 = bi + wi + 32 * x + 4 * h, j = bj + wj + 32 * y + li;
+            float own[16];
+            if (MODE == kFull && g.accumulate) {
+                // All 16 requested before the first store (clamped: what lies past an edge is not stored).
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    own[r] = g.c[(size_t)min(i0 + (r & 3) + 8 * (r >> 2), M - 1) * g.ldc + min(j, N - 1)];
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int i = bi + wi + 32 * x + (r & 3) + 8 * (r >> 2) + 4 * h, j = bj + wj + 32 * y + li;
+                const int i = i0 + (r & 3) + 8 * (r >> 2);
                 if (i >= M || j >= N) continue;
                 if constexpr (MODE == kUpperReversed) {
                     if (j >= i) g.c[(size_t)(M - 1 - i) * g.ldc + (N - 1 - j)] = (float)sum[x][y][r];
                 } else {
                     const float v = g.alpha * acc[x][y][r];
-                    float *p = g.c + (size_t)i * g.ldc + j;
-                    *p = g.accumulate ? *p + v : v;
+                    g.c[(size_t)i * g.ldc + j] = g.accumulate ? own[r] + v : v;
                 }
             }
+        }
 }
 
 template <int TA, int TB>
