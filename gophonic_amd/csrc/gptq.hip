@@ -15,8 +15,10 @@
 //     choosing each 4-bit group's scale (q4GroupScale) from the current values
 //     at the group's first column; then the columns after the block take the
 //     lazy update W -= E U (an fp32 product).
-// All products are fp32 with fp32 storage, as the reference's; the small
-// substitutions sum in float64, as the reference's do.
+// Storage is fp32, as the reference's. The Gram matrix adds each 16-row chunk's
+// fp32 sum in float64, the factorization works within a panel in float64 (the
+// reference's substitutions sum in float64), the trailing products and the lazy
+// updates are fp32 products with fp32 sums.
 #include <math.h>
 
 #include <algorithm>
@@ -155,11 +157,11 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
     sgemm_stash<TB ^ 1, BN>(Bs[0], vb);
     __syncthreads();
     int buf = 0;
-    for (int p0 = 0; p0 < K; p0 += 16) {
-        const bool more = p0 + 16 < K;
+    for (uint32_t p0 = 0; p0 < (uint32_t)K; p0 += 16) {  // unsigned: K may be INT32_MAX
+        const bool more = p0 + 16 < (uint32_t)K;
         if (more) {
-            sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, p0 + 16, g.vecA);
-            sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, p0 + 16, g.vecB);
+            sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, (int)p0 + 16, g.vecA);
+            sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, (int)p0 + 16, g.vecB);
         }
 #pragma unroll
         for (int gr = 0; gr < 2; ++gr) {
