@@ -292,13 +292,13 @@ __global__ __launch_bounds__(64 * SK) void vecd_kernel(const Vec2Args a) {
 }
 
 // How a vecs_kernel launch cuts K: `parts` passes over the block's row tiles,
-// each over SK wavefronts' slices of NB 32-value blocks.
+// each over SK wavefronts' slices of nb 32-value blocks.
 struct VecsShape {
-    int iters, SK, parts;
+    int iters, SK, nb, parts;
     int svec;  // block scales load as one aligned vector per lane
 };
 
-// NB: 32-value blocks per slice (their A fragments stay in registers).
+// NB: 32-value blocks per slice, at most (their A fragments stay in registers).
 template <int FMT, int T, bool PAIR, int NB>
 struct VecsTraits {
     static constexpr bool Q4 = FMT == GPHQ_FMT_Q4;
@@ -329,9 +329,9 @@ struct VecsTraits {
 // turn into B fragments through the wavefront's LDS, the next tile's loads in
 // flight meanwhile. Slices meet in LDS, a few tiles at a time. K past one
 // pass's slices takes further passes over the same tiles, whose sums wait in
-// LDS. 8 vectors, Q4, K = 4096, N = 24576: 65.4 -> 20.7
-// us with its preparation; 32 vectors 101.8 -> 44.8, 8 vectors at K = 12288, N =
-// 4096 35.3 -> 18.2.
+// LDS. 8 vectors, Q4, K = 4096, N = 24576: 65.6 -> 18.5 us with its preparation
+// (VALU busy 34%, 3.5 TB/s); 32 vectors 102 -> 46.4, 8 vectors at K = 12288, N =
+// 4096 35.1 -> 16.4.
 template <int FMT, int T, bool PAIR, int NB, int EPI, bool NORM>
 __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void vecs_kernel(const Vec2Args a,
                                                                                              const VecsShape sh) {
@@ -345,7 +345,7 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
     const int lane = threadIdx.x & 63;
     const int ks = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int g = lane >> 4, m = lane & 15;
-    const int KB = a.KB, SK = sh.SK, iters = sh.iters, CH = X::ch(SK);
+    const int KB = a.KB, SK = sh.SK, nb = sh.nb, iters = sh.iters, CH = X::ch(SK);
     u32x4 *const st = (u32x4 *)(smem + ks * X::kWave);
     uint8_t *const ssc = smem + ks * X::kWave + X::kStage;
     float *const siv = (float *)(ssc + X::kScale);
@@ -427,8 +427,8 @@ __global__ __launch_bounds__((64 * VecsTraits<FMT, T, PAIR, NB>::kMaxSK)) void v
         }
     };
     for (int part_i = 0; part_i < sh.parts; ++part_i) {
-        kb0 = min((part_i * SK + ks) * NB, KB);
-        const int mine = min(NB, KB - kb0);  // blocks of this slice (0: none left)
+        kb0 = min((part_i * SK + ks) * nb, KB);
+        const int mine = min(nb, KB - kb0);  // blocks of this slice (0: none left)
         int tt = blockIdx.x;
         gload(tt);
         // All of the slice's activation loads are issued before the first is used.
@@ -959,7 +959,9 @@ size_t gemv_vec_workspace_bytes(int V, int K) {
 
 // The slices of K: as few passes as hold KB blocks, each over as few wavefronts
 // as hold a pass's share (twice the wavefronts at half the blocks each took
-// 8 vectors, K = 1376, N = 24000, Q8B 17.7 us, 14.4 with this). Where the tiles'
+// 8 vectors, K = 1376, N = 24000, Q8B 17.7 us, 14.4 with this), or as many more
+// as leave as many blocks on a CU (16 vectors, K = 4128, N = 20000, Q8B, six
+// slices of 12 blocks instead of five of 16: 46.7 -> 44.5 us). Where the tiles'
 // sums of a further pass would not fit in LDS, more blocks walk fewer tiles.
 template <int FMT, int T, bool PAIR, int NB, int EPI, bool NORM>
 static int go_vecs(const Vec2Args &a, hipStream_t stream) {
@@ -968,10 +970,15 @@ static int go_vecs(const Vec2Args &a, hipStream_t stream) {
     VecsShape sh{};
     sh.parts = (a.KB + kMaxSK * NB - 1) / (kMaxSK * NB);
     const int per = (a.KB + sh.parts - 1) / sh.parts;  // blocks of one pass
-    sh.SK = (per + NB - 1) / NB;
+    const int line = X::Q4 ? 8 : 4;  // blocks per 128-byte line
+    constexpr int kWaves = T == 1 && !PAIR ? kMaxSK : 8;  // wavefronts per CU
+    const int least = (per + NB - 1) / NB, perCu = std::max(1, kWaves / least);
+    sh.nb = std::min(NB, ((per + kWaves / perCu - 1) / (kWaves / perCu) + line - 1) / line * line);
+    if (least > kWaves) sh.nb = NB;
+    sh.SK = (per + sh.nb - 1) / sh.nb;
     sh.svec = X::SB && a.KB % 4 == 0 && (uintptr_t)a.scales % 16 == 0;
     const int tiles = (a.N + 15) / 16;
-    int blocks = std::max(1, std::min(tiles, device_cus() * std::max(1, (T == 1 && !PAIR ? kMaxSK : 8) / sh.SK)));
+    int blocks = std::max(1, std::min(tiles, device_cus() * perCu));
     sh.iters = (tiles + blocks - 1) / blocks;
     const int room = (kLds - X::lds(sh.SK, 1, 0)) / (T * 1024);
     if (sh.parts > 1 && sh.iters > room) sh.iters = room;
