@@ -11,15 +11,20 @@
 // a single contiguous 1 KiB wavefront load. Padding (rows past R, K past the
 // logical K) is zero in the weights, so padded K never changes a sum.
 //
-// GEMM: a block is WM x WN x SK wavefronts; wavefront (wm, wn, ks) owns a
-// (16*TM) x (16*TN) output tile and the ks-th slice of the K tiles. It loads
-// U K-steps of A and B fragments straight from HBM/L2 into registers, then
-// issues TM*TN MFMAs per step. With SK > 1 the int32 partial tiles are added
-// in LDS (exact, so any split gives identical bits). The epilogue converts
-// int32 -> fp32 (round to nearest even, like Go's float32(int32)) and applies
-// the two scale multiplies in the reference's order. Blocks are renumbered so
-// that consecutive blocks on one XCD share a weight column tile, which is then
-// read from HBM once into that XCD's L2.
+// GEMM kernels, all exact in int32 and with one epilogue (int32 -> fp32 rounded
+// to nearest even, like Go's float32(int32), then the two scale multiplies in the
+// reference's order), so any of them gives the same bits:
+//   * i8gemm_kernel (up to 16 rows): fragments straight from HBM / L2 into
+//     registers, K split over a block's wavefronts, whose int32 partial tiles are
+//     added in LDS;
+//   * i8gemm_roles_kernel: tiles of 16 x 16 to 128 x 192, loading and multiplying
+//     wavefronts apart, operands direct to a ring of LDS stages; tile layout or
+//     the batched pass's row tiles and row-major weights;
+//   * i8gemm_pp_kernel (tile layout) and i8gemm_rows_kernel (batched pass): 256-row
+//     tiles, two groups of wavefronts half a K-step apart.
+// i8gemm_launch and lm_i8_mm choose by rounds of the chip. Blocks are renumbered
+// (tile_order, and by hand in i8gemm_kernel) so that consecutive blocks of one XCD
+// share weight columns, which that XCD's L2 then reads once.
 #include "common.h"
 
 namespace gphq {
@@ -348,9 +353,12 @@ struct I8GemmArgs {
     int K;             // row length in bytes of row-major weights (a multiple of 64)
 };
 
-// Operand layouts and epilogues of the big-tile kernel.
+// Epilogues: store, fp32 add into dst, SwiGLU of interleaved columns.
 enum { I8_EPI_STORE = 0, I8_EPI_ADD = 1, I8_EPI_SWIGLU = 2 };
 
+// A block is WM x WN x SK wavefronts; wavefront (wm, wn, ks) owns a (16 TM) x (16
+// TN) output tile and the ks-th slice of the K tiles. It loads U K-steps of A and
+// B fragments into registers, then issues TM TN MFMAs per step.
 template <int TM, int TN, int WM, int WN, int SK, int U>
 __global__ __launch_bounds__(64 * WM * WN * SK) void i8gemm_kernel(const I8GemmArgs a) {
     constexpr int NW = WM * WN * SK;
@@ -471,12 +479,6 @@ __global__ __launch_bounds__(64 * WM * WN * SK) void i8gemm_kernel(const I8GemmA
     }
 }
 
-// Epilogue of the direct-to-LDS kernels, as in i8gemm_kernel: lane l of a
-// 16 x 16 tile holds rows 4 (l / 16) + e, column l % 16; scales first, then
-// the stores. mt0 / nt0: the wavefront's first row and column tile.
-// Measured on MI355X (config 2, M = 512): stores of 16 columns per row wrote
-// 1.32x the output's bytes to HBM (WRITE_SIZE); whole 128-byte lines write
-// them once.
 // The stores of dma_epilogue with the column-tile pairs starting at tile P
 // of the wavefront (P = nt0 % 2, so that each pair's 32 columns are one
 // 128-byte line of every row): v_permlane16_swap exchanges lanes 16-31 of
@@ -711,9 +713,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void i8gemm_pp_kernel(const I8GemmA
 
 // The ping-pong schedule for row-major weights (the batched pass): a 64-deep
 // step takes half a 128-byte line of each weight row, and loads of half lines
-// (16 rows x 64 bytes an instruction) held the schedule to 1.67 POPS (Qwen3-8B
-// gate/up at 4096 rows, SwiGLU; the tile layout's whole groups run 2.58). Whole
-// lines: 498 -> 465 us with the activation pack, 1.85 POPS. B comes in pieces
+// (16 rows x 64 bytes an instruction) held the schedule to 1.75 POPS (472 us, Qwen3-
+// 8B gate/up at 4096 rows, SwiGLU; the tile layout's whole groups run 2.58 with a
+// plain store). Whole lines: 445 us, 1.85 POPS; with the activation pack (26 us)
+// 498 -> 463 us. MFMA busy 41%, VALU busy 43%. B comes in pieces
 // of two K-steps: 8 rows x 128 bytes an instruction, lane l taking chunk (l % 8)
 // ^ ((row / 2) % 8) of row l / 8, so that a fragment's 16 rows at one chunk sit on distinct
 // banks. LDS holds four A stages and three B pieces; a step requests A's stage
@@ -1007,7 +1010,12 @@ int i8gemm_launch(const int8_t *A, const int8_t *B, const float *rowScale, const
     // 14.2 / 19.6 / 23.8 / 35.9 / 75.3 / 387 us before (tiles chosen by M
     // alone, each wavefront loading what it multiplies), 12.5 / 13.0 / 15.9 /
     // 20.0 / 30.8 / 47.7 / 160 with this; N = 3396: 12.2 / 12.9 / 18.1 / 21.8 /
-    // 31.4 / 41.0 / 122 before, 9.3 / 9.4 / 12.1 / 12.8 / 16.2 / 22.1 / 55.6.
+    // 31.4 / 41.0 / 122 before, 9.3 / 9.4 / 12.1 / 12.8 / 16.2 / 22.1 / 55.6
+    // (weights from the 256 MB cache). With weights that no cache holds, over 506
+    // sizes (17-1500 rows, K = 64 to 8192, N = 594 to 12288) the tile taken is 0.9%
+    // behind the fastest on average; 25 sizes lose more than 6%, most at 896 x
+    // 7040 -> 10234 (107 us in 128 x 96, 68 in 256 x 256); 20 rows, 4096 ->
+    // 12288, take 12.7 us (12.3 before).
     struct Tile {
         int bm, bn, ns;
     };
@@ -1081,11 +1089,6 @@ int lm_i8_act(const float *x, long stride, int rows, int K, bool norm, float eps
     return launch_i8_act_rows<1, false>(x, stride, rows, K, eps, nullptr, 0, act, rowScale, stream);
 }
 
-// One projection of the batched pass on the int8 route: y = (float32(A W^T)
-// * w_scale) * a_scale for int8 activations A in row tiles (lm_i8_act)
-// and row-major Q8 codes W [N][K] (one fp32 scale per weight row), then epi 0
-// stores y[M][N], 1 adds it into y, 2 stores the SwiGLU of interleaved gate/up
-// columns into y[M][N/2]; y rows are y_stride floats apart. K % 64 == 0.
 // The batched pass's int8 GEMM over columns [a.c0, a.c1) in 256 x BN tiles.
 template <int BN>
 static int lm_i8_mm_rows(int epi, const I8GemmArgs &a, hipStream_t stream) {
@@ -1101,6 +1104,11 @@ static int lm_i8_mm_roles(int epi, const I8GemmArgs &a, hipStream_t stream) {
     return launch_i8gemm_roles<BM, BN, WGM, WGN, NP, SB, NS, true, I8_EPI_SWIGLU>(a, stream);
 }
 
+// One projection of the batched pass on the int8 route: y = (float32(A W^T)
+// * w_scale) * a_scale for int8 activations A in row tiles (lm_i8_act)
+// and row-major Q8 codes W [N][K] (one fp32 scale per weight row), then epi 0
+// stores y[M][N], 1 adds it into y, 2 stores the SwiGLU of interleaved gate/up
+// columns into y[M][N/2]; y rows are y_stride floats apart. K % 64 == 0.
 int lm_i8_mm(int epi, const int8_t *act, const float *a_scale, const int8_t *codes, const float *w_scale, float *y,
              long y_stride, int M, int K, int N, hipStream_t stream) {
     if (M == 0 || N == 0) return GPHQ_OK;
