@@ -1022,8 +1022,10 @@ static int launch_vecs_tiles(const Vec2Args &a, hipStream_t stream) {
 // 5.1 / 5.8, 928 -> 6144 7.3 / 6.8; 32 vectors, Q8B, 928 -> 4096 8.8 / 10.0,
 // 3168 -> 5000 35.8 / 25.5; 17 vectors, Q4, one whole pass, 2048 -> 6144 16.7 /
 // 12.2, one block more, 2080 -> 5000 15.0 / 16.4. 64-row blocks of eight slices:
-// 17-24 vectors just past one pass (Q4, 2080 -> 16000: 21.8 / 26.1), as long as
-// they are one round of the chip (24000: 36.5 / 35.6; Q8B_F32, 2336 -> 16000: 28.6 / 24.8).
+// 17-24 vectors just past one pass (Q4, 2080 -> 16000: 21.8 / 26.1) and row-scaled
+// codes wherever a pass is not nearly full (Q8, 31 vectors, 6208 -> 14000 59.5 /
+// 66.0; 10240 -> 14000, full passes, 86.6 / 89.2), as long as they are one round
+// of the chip (Q4, 2080 -> 24000: 36.5 / 35.6; Q8B_F32, 2336 -> 16000: 28.6 / 24.8).
 static int vecd_rows(int fmt, int V, int KB, int N) {
     static constexpr struct {
         int onePass, perPass, work, maxTiles;
@@ -1033,8 +1035,9 @@ static int vecd_rows(int fmt, int V, int KB, int N) {
     const auto &r = kRules[V <= 8 ? 0 : V <= 16 ? 1 : 2][fmt == GPHQ_FMT_Q8 ? 0 : fmt == GPHQ_FMT_Q4 ? 2 : 1];
     const long tiles = ((long)N + 15) / 16;
     const int pass = V > 16 ? 64 : 128, parts = (KB + pass - 1) / pass;
-    if (V > 16 && V <= 24 && fmt != GPHQ_FMT_Q8B_F32 && KB > pass && KB <= 80 && tiles > 2 * device_cus() &&
-        tiles <= 4 * device_cus())
+    const bool oneRound = tiles > 2 * device_cus() && tiles <= 4 * device_cus();  // of 64-row blocks
+    if (V > 16 && KB > pass && oneRound &&
+        (fmt == GPHQ_FMT_Q8 ? KB <= 56 * parts : V <= 24 && KB <= 80 && fmt != GPHQ_FMT_Q8B_F32))
         return 64;
     const bool few = parts == 1 ? KB <= r.onePass : parts <= 3 && KB <= r.perPass * parts;
     return few && KB * tiles <= r.work && tiles <= r.maxTiles ? 16 : 0;
@@ -1042,7 +1045,7 @@ static int vecd_rows(int fmt, int V, int KB, int N) {
 
 template <int FMT, int MT, int EPI, bool NORM>
 static int go_vecd(const Vec2Args &a, int rows, hipStream_t stream) {
-    if constexpr (MT == 3) {
+    if constexpr (MT == 3 || (MT == 4 && FMT == GPHQ_FMT_Q8)) {
         if (rows == 64) {
             hipLaunchKernelGGL((vecd_kernel<FMT, MT, 8, 4, 2, EPI, NORM>), dim3((unsigned)((a.N + 63) / 64)), dim3(512),
                                0, stream, a);

@@ -135,7 +135,7 @@ def test_slice_and_pass_edges(fmt, k, n):
     # more tiles a block than its LDS holds between passes
     (orc.FMT_Q4, 32, 3648, 75000),
     # 64-row blocks, the last one cut
-    (orc.FMT_Q8, 17, 2080, 16000), (orc.FMT_Q8B, 24, 2336, 9001),
+    (orc.FMT_Q8, 17, 2080, 16000), (orc.FMT_Q8B, 24, 2336, 9001), (orc.FMT_Q8, 31, 6208, 11822),
     # few rows past the small products' sizes: partial last slices and passes
     (orc.FMT_Q8, 5, 1700, 17), (orc.FMT_Q8, 17, 4256, 1), (orc.FMT_Q8B, 9, 1248, 40), (orc.FMT_Q8B_F32, 32, 2720, 33),
     (orc.FMT_Q4, 2, 608, 100), (orc.FMT_Q4, 12, 8256, 31),
