@@ -1022,10 +1022,13 @@ static int launch_vecs_tiles(const Vec2Args &a, hipStream_t stream) {
 // 5.1 / 5.8, 928 -> 6144 7.3 / 6.8; 32 vectors, Q8B, 928 -> 4096 8.8 / 10.0,
 // 3168 -> 5000 35.8 / 25.5; 17 vectors, Q4, one whole pass, 2048 -> 6144 16.7 /
 // 12.2, one block more, 2080 -> 5000 15.0 / 16.4. 64-row blocks of eight slices:
-// 17-24 vectors just past one pass (Q4, 2080 -> 16000: 21.8 / 26.1) and row-scaled
-// codes wherever a pass is not nearly full (Q8, 31 vectors, 6208 -> 14000 59.5 /
-// 66.0; 10240 -> 14000, full passes, 86.6 / 89.2), as long as they are one round
-// of the chip (Q4, 2080 -> 24000: 36.5 / 35.6; Q8B_F32, 2336 -> 16000: 28.6 / 24.8).
+// 17-24 vectors just past one pass (Q4, 2080 -> 16000: 21.8 / 26.1), and row-
+// scaled codes, whose widening and adding is most of vecs_kernel's time when the
+// weights come from the 256 MB cache (Q8, 31 vectors, 12288 -> 14000: 80 / 106 us
+// cached, 101 / 106 not; 6208 -> 14000 59.5 / 66.0 not), except where its passes
+// are nearly full and the rows few (8192 -> 11822: 59.1 / 61.6 cached, 72.1 / 62.5
+// not), as long as they are one round of the chip (Q4, 2080 -> 24000: 36.5 / 35.6;
+// Q8B_F32, 2336 -> 16000: 28.6 / 24.8).
 static int vecd_rows(int fmt, int V, int KB, int N) {
     static constexpr struct {
         int onePass, perPass, work, maxTiles;
@@ -1037,7 +1040,8 @@ static int vecd_rows(int fmt, int V, int KB, int N) {
     const int pass = V > 16 ? 64 : 128, parts = (KB + pass - 1) / pass;
     const bool oneRound = tiles > 2 * device_cus() && tiles <= 4 * device_cus();  // of 64-row blocks
     if (V > 16 && KB > pass && oneRound &&
-        (fmt == GPHQ_FMT_Q8 ? KB <= 56 * parts : V <= 24 && KB <= 80 && fmt != GPHQ_FMT_Q8B_F32))
+        (fmt == GPHQ_FMT_Q8 ? KB <= 56 * parts || parts > 4 || tiles > 3 * device_cus()
+                            : V <= 24 && KB <= 88 && fmt != GPHQ_FMT_Q8B_F32))
         return 64;
     const bool few = parts == 1 ? KB <= r.onePass : parts <= 3 && KB <= r.perPass * parts;
     return few && KB * tiles <= r.work && tiles <= r.maxTiles ? 16 : 0;
