@@ -157,11 +157,13 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
     sgemm_stash<TB ^ 1, BN>(Bs[0], vb);
     __syncthreads();
     int buf = 0;
-    for (uint32_t p0 = 0; p0 < (uint32_t)K; p0 += 16) {  // unsigned: K may be INT32_MAX
-        const bool more = p0 + 16 < (uint32_t)K;
+    // Chunks are counted: K may be INT32_MAX, and a position past the last chunk would not fit.
+    const int chunks = (int)(((uint32_t)K + 15) / 16);
+    for (int chunk = 1; chunk <= chunks; ++chunk) {
+        const bool more = chunk < chunks;
         if (more) {
-            sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, (int)p0 + 16, g.vecA);
-            sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, (int)p0 + 16, g.vecB);
+            sgemm_fetch<TA, BM>(va, g.a, g.lda, M, K, bi, chunk * 16, g.vecA);
+            sgemm_fetch<TB ^ 1, BN>(vb, g.b, g.ldb, N, K, bj, chunk * 16, g.vecB);
         }
 #pragma unroll
         for (int gr = 0; gr < 2; ++gr) {
@@ -200,9 +202,18 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
     for (int x = 0; x < MT; ++x)
 #pragma unroll
         for (int y = 0; y < NT; ++y) {
+            if constexpr (MODE == kUpperReversed) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int i = bi + wi + 32 * x + (r & 3) + 8 * (r >> 2) + 4 * h, j = bj + wj + 32 * y + li;
+                    if (i < M && j < N && j >= i)
+                        g.c[(size_t)(M - 1 - i) * g.ldc + (N - 1 - j)] = (float)sum[x][y][r];
+                }
+                continue;
+            }
             const int i0 = bi + wi + 32 * x + 4 * h, j = bj + wj + 32 * y + li;
             float own[16];
-            if (MODE == kFull && g.accumulate) {
+            if (g.accumulate) {
                 // All 16 requested before the first store (clamped: what lies past an edge is not stored).
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
@@ -212,12 +223,8 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmArgs g) {
             for (int r = 0; r < 16; ++r) {
                 const int i = i0 + (r & 3) + 8 * (r >> 2);
                 if (i >= M || j >= N) continue;
-                if constexpr (MODE == kUpperReversed) {
-                    if (j >= i) g.c[(size_t)(M - 1 - i) * g.ldc + (N - 1 - j)] = (float)sum[x][y][r];
-                } else {
-                    const float v = g.alpha * acc[x][y][r];
-                    g.c[(size_t)i * g.ldc + j] = g.accumulate ? own[r] + v : v;
-                }
+                const float v = g.alpha * acc[x][y][r];
+                g.c[(size_t)i * g.ldc + j] = g.accumulate ? own[r] + v : v;
             }
         }
 }
@@ -286,12 +293,23 @@ using f64x4 = __attribute__((ext_vector_type(4))) double;
 
 // Lane N's value in each row of 16 lanes (DPP row_newbcast).
 template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + N, 0xF, 0xF, true));
+}
+template <int N>
 __device__ __forceinline__ double row_bcast(double v) {
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
     const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, 0x150 + N, 0xF, 0xF, true);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), 0x150 + N, 0xF, 0xF, true);
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
+
+// A value of the diagonal block. An infinite pivot (an overflowed Gram matrix) is
+// the reference's sqrt(Inf): Inf on the diagonal, zeros below it and in the
+// inverse. As 1e300, from which updates take nothing, it gives the same float32
+// values without Inf * 0 on the way (an infinity off the diagonal still ends in a
+// pivot that is not positive, and a NaN stays one).
+__device__ __forceinline__ double diag_value(float v) { return v > 3.4028235e38f ? 1e300 : (double)v; }
 
 // The diagonal block's working storage: D's lower 16 x 16 blocks hold A, then
 // L; an upper block (c, r) holds block (r, c) of S, then of L^-1, transposed;
@@ -318,10 +336,7 @@ __device__ __forceinline__ void chol16_steps(double (&a)[16], double (&w)[4], in
         double d = row_bcast<J>(a[J]);
         const bool positive = d > 0.0;
         fail = fail || !positive;
-        // An infinite pivot (an overflowed Gram matrix) is the reference's
-        // sqrt(Inf): Inf on the diagonal, zeros below it and in the inverse.
-        // Bounded here it gives the same float32 values without Inf * 0 below.
-        d = positive ? fmin(d, 1e300) : 1.0;
+        d = positive ? d : 1.0;
         // sqrt(d) and its reciprocal from the hardware's estimate, two Goldschmidt steps.
         double r = __builtin_amdgcn_rsq(d), piv = d * r, hr = 0.5 * r;
 #pragma unroll
@@ -332,12 +347,13 @@ __device__ __forceinline__ void chol16_steps(double (&a)[16], double (&w)[4], in
         }
         r = 2.0 * hr;
         // choleskyLower's column (gptq_linalg.go:73-93), stored as float32.
-        const double l = (double)(i == J ? (float)piv : (float)(a[J] * r));
+        const float lf = i == J ? (float)piv : (float)(a[J] * r);
+        const double l = (double)lf;
         a[J] = l;
         const double li = i > J ? l : 0.0;
         chol16_row<J, J + 1>(a, l, li);
         // The reciprocal of the stored pivot; row J of the inverse is final.
-        const double ljj = fmin(row_bcast<J>(l), 1e150);
+        const double ljj = (double)fminf(row_bcast<J>(lf), 3.4028235e38f);  // finite
 #pragma unroll
         for (int n = 0; n < 2; ++n) r = fma(r, fma(-ljj, r, 1.0), r);
         const double lr = li * r;
@@ -465,7 +481,7 @@ __global__ __launch_bounds__(256, 3) void chol_first_kernel(float *a, int n, flo
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
         const int e = (int)threadIdx.x + 256 * u, r = e >> 6, c = e & 63;
-        d.D[r][c] = r < b && c <= r ? (double)v[u] : r == c ? 1.0 : 0.0;
+        d.D[r][c] = r < b && c <= r ? diag_value(v[u]) : r == c ? 1.0 : 0.0;
     }
     __syncthreads();
     chol_diag(d, b, a, x, n, inv, bad);
@@ -620,7 +636,7 @@ __global__ __launch_bounds__(256, 3) void chol_update_kernel(float *a, int n, in
         const int lr = wi + (r & 3) + 8 * (r >> 2) + 4 * h, lc = wj + li;
         const float v = trailing ? own[r] - acc[r] : fresh ? acc[r] : own[r] + acc[r];
         // Past the matrix's edge the diagonal block continues as the identity.
-        if (diag) sh.d.D[lr][lc] = bi + lr < n ? (double)v : lr == lc ? 1.0 : 0.0;
+        if (diag) sh.d.D[lr][lc] = bi + lr < n ? diag_value(v) : lr == lc ? 1.0 : 0.0;
         else if (bi + lr < n && bj + lc <= bi + lr) c[(size_t)(bi + lr) * n + bj + lc] = v;
     }
     if (!diag) return;
